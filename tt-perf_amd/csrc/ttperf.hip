@@ -996,6 +996,18 @@ int ensure_staging(ttp_ctx* c, uint64_t bytes) {
 // this many elements (64 MiB of fp32).
 constexpr uint64_t kPieceElems = 16ull << 20;
 
+// Whether a slot transfer runs four elements per lane: the contiguous array is 16-byte aligned
+// (a caller's device pointer may be any fp32 element's address) and the slot's range starts on a
+// record (tensors and staged pieces do).  Faster at every size measured (see
+// gather_slot4_kernel), so the one-element kernels keep the other pointers only.
+bool slot_words(uint64_t first, const void* p) {
+    return ((uintptr_t)p & 15u) == 0 && first % ttp::kRec == 0;
+}
+uint64_t slot_blocks(uint64_t n) {
+    const uint64_t per = ttp::kSlotLanes * ttp::kSlotElems;
+    return (n + per - 1) / per;
+}
+
 // slot elements [first, first + n) of record-stored buffer `which` -> contiguous device array
 // (a BF16 store's checkpoint master: its bf16 weights, widened exactly)
 int gather_slot(ttp_ctx* c, int which, uint64_t first, uint64_t n, float* dst) {
@@ -1008,9 +1020,16 @@ int gather_slot(ttp_ctx* c, int which, uint64_t first, uint64_t n, float* dst) {
         HIP_TRY(hipGetLastError());
         return TTP_OK;
     }
-    hipLaunchKernelGGL(ttp::gather_slot_kernel, dim3(elementwise_grid(c, n)), dim3(ttp::kBlock),
-                       0, c->stream, (const float*)buffer_base(c, which),
-                       buffer_stride(c, which), first, n, dst);
+    const float* slot = (const float*)buffer_base(c, which);
+    const uint32_t stride = buffer_stride(c, which);
+    if (slot_words(first, dst))
+        launch_lanes(c, slot_blocks(n), ttp::kSlotLanes, [&](dim3 g, uint64_t b0) {
+            hipLaunchKernelGGL(ttp::gather_slot4_kernel, g, dim3(ttp::kSlotLanes), 0, c->stream,
+                               slot, stride, first, n, dst, b0);
+        });
+    else
+        hipLaunchKernelGGL(ttp::gather_slot_kernel, dim3(elementwise_grid(c, n)),
+                           dim3(ttp::kBlock), 0, c->stream, slot, stride, first, n, dst);
     HIP_TRY(hipGetLastError());
     return TTP_OK;
 }
@@ -1033,9 +1052,20 @@ int scatter_slot(ttp_ctx* c, int which, uint64_t first, uint64_t n, const float*
     uint16_t* p16 = (c->mode == TTP_MODE_MIXED && which == TTP_BUF_MASTER) ? (uint16_t*)c->param
                                                                           : nullptr;
     clear_hip_error();
-    hipLaunchKernelGGL(ttp::scatter_slot_kernel, dim3(elementwise_grid(c, n)), dim3(ttp::kBlock),
-                       0, c->stream, (float*)buffer_base(c, which), buffer_stride(c, which),
-                       first, n, src, p16);
+    float* slot = (float*)buffer_base(c, which);
+    const uint32_t stride = buffer_stride(c, which);
+    if (src && slot_words(first, src))
+        launch_lanes(c, slot_blocks(n), ttp::kSlotLanes, [&](dim3 g, uint64_t b0) {
+            if (p16)
+                hipLaunchKernelGGL(ttp::scatter_slot4_kernel<true>, g, dim3(ttp::kSlotLanes), 0,
+                                   c->stream, slot, stride, first, n, src, p16, b0);
+            else
+                hipLaunchKernelGGL(ttp::scatter_slot4_kernel<false>, g, dim3(ttp::kSlotLanes), 0,
+                                   c->stream, slot, stride, first, n, src, p16, b0);
+        });
+    else
+        hipLaunchKernelGGL(ttp::scatter_slot_kernel, dim3(elementwise_grid(c, n)),
+                           dim3(ttp::kBlock), 0, c->stream, slot, stride, first, n, src, p16);
     HIP_TRY(hipGetLastError());
     return TTP_OK;
 }
