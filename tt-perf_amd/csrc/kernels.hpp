@@ -1,15 +1,13 @@
 // kernels.hpp — gfx950 device code of libttperf_hip.
 //
-// One optimizer step over the flat store is at most four launches on one stream:
+// One optimizer step over the flat store is at most three launches on one stream:
 //   norm_partials_kernel  reads only the gradients (2 B/param bf16, 4 B/param fp32) in 16 KiB
 //                         tiles: fp64 sum of squares of the unscaled grads, one partial per
-//                         block; no atomics and no fences (a per-block device-scope fence +
-//                         ticket costs ~50 ns per block on MI355X, serialised, which tripled
-//                         the pass's time).  Two launches above 256 MiB of gradients:
-//                         non-temporal loads, then cached loads for the last 256 MiB;
-//   norm_finalize_kernel  one block: sums the partials in index order (deterministic),
-//                         decides found_inf / skip and the clip coefficient, advances the step
-//                         count and the loss scale;
+//                         block; the last block to finish sums the partials in index order
+//                         (deterministic), decides found_inf / skip and the clip coefficient,
+//                         advances the step count and the loss scale.  Two launches above
+//                         256 MiB of gradients: non-temporal loads, then cached loads for the
+//                         last 256 MiB;
 //   adam_lane_kernel /    one fused pass per element: grad transform (unscale, clip), weight
 //   sgd_lane_kernel       decay, the optimizer update and the bf16 copy, one or two elements
 //                         per lane; sgd_kernel does the same with four elements per lane
@@ -196,110 +194,7 @@ __device__ __forceinline__ double block_sum(double x, double* lds) {
 }
 
 // ------------------------------------------------------------------------------------
-// norm pass, part 1: per-block partial sums of squares of the unscaled gradients
-// ------------------------------------------------------------------------------------
-// 16-byte loads: 8 bf16 or 4 fp32 gradients per lane
-template <typename GradT>
-struct GradVec;
-template <>
-struct GradVec<uint16_t> {
-    static constexpr int kElems = 8;
-    typedef uint32_t raw __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ float at(const raw& w, int j) {
-        return (j & 1) ? bf16_hi(w[j >> 1]) : bf16_lo(w[j >> 1]);
-    }
-    // element j of a vector that starts as zeros
-    static __device__ __forceinline__ void put(raw& w, int j, uint16_t h) {
-        w[j >> 1] |= (j & 1) ? ((uint32_t)h << 16) : (uint32_t)h;
-    }
-};
-template <>
-struct GradVec<float> {
-    static constexpr int kElems = 4;
-    typedef f32x4 raw;
-    static __device__ __forceinline__ float at(const raw& w, int j) { return w[j]; }
-    static __device__ __forceinline__ void put(raw& w, int j, float x) { w[j] = x; }
-};
-
-// Norm tiles: kNormLoads 16-byte loads per lane, so a tile is 16 KiB of gradients (8192 bf16
-// or 4096 fp32); the pass has its own tile table (same tensors, bigger pieces than the update's
-// chunks) so each descriptor fetch is amortised over 4 loads per lane.
-constexpr int kNormLoads = 4;
-template <typename GradT>
-constexpr uint32_t norm_tile_elems() {
-    return (uint32_t)(kBlock * kNormLoads * 16 / sizeof(GradT));
-}
-
-// Grid-stride over the norm tiles t0 .. t1-1, one partial per block.  A whole tile (every tile
-// but a tensor's last) is four unconditional 16-byte loads per lane, all issued before the
-// arithmetic (the scheduling barrier keeps the compiler from interleaving them with it, which
-// left one or two loads in flight: 6.0-6.3 TB/s against 6.7-6.9 at GPT-2 774M / 1558M).
-// kNT selects non-temporal loads.  The host runs the pass as two launches: non-temporal over
-// all but the last kCachedGradBytes of gradients, then cached loads over those, which the
-// update, walking the chunks in reverse, reads first and so finds in the 256 MB Infinity
-// Cache (measured on GPT-2 124M: update 531 us after this pass vs 559 us alone; at 774M and
-// 1558M fp32 the split pass runs 232 and 931 us against 246-260 and 978-1030 us with cached
-// loads throughout, the update unchanged).  No atomics and no fences: each block writes one
-// partial and norm_finalize_kernel (next on the stream) combines them.  Squares of fp32
-// values are exact in fp64, and any inf/NaN gradient makes the sum non-finite.
-template <typename GradT, bool kNT>
-__global__ __launch_bounds__(kBlock) void norm_partials_kernel(const GradT* __restrict__ g,
-                                                               const Chunk* __restrict__ tiles,
-                                                               uint32_t t0, uint32_t t1,
-                                                               const DevState* __restrict__ st,
-                                                               int32_t scaler_on,
-                                                               double* __restrict__ partials) {
-    typedef GradVec<GradT> GV;
-    typedef typename GV::raw R;
-    constexpr int E = GV::kElems;
-    constexpr uint32_t kTile = norm_tile_elems<GradT>();
-    __shared__ double lds[kBlock / 64];
-    const float inv = scaler_on ? (float)(1.0 / (double)st->scale) : 1.0f;
-    // two accumulators (element j of a vector goes to acc[j & 1]): a fixed order, so the
-    // sum stays deterministic, with half the dependent-add chain.  The square of an fp32 value
-    // is exact in fp64, so fma(x, x, acc) rounds exactly as acc + x*x does (one rounding, of
-    // the add) with one instruction instead of two.
-    double acc[2] = {0.0, 0.0};
-    for (uint32_t c = t0 + blockIdx.x; c < t1; c += gridDim.x) {
-        const Chunk ch = load_chunk(tiles, c);
-        const R* q = reinterpret_cast<const R*>(g + ch.begin) + threadIdx.x;
-        if (ch.count == kTile) {
-            R w[kNormLoads];
-#pragma unroll
-            for (int l = 0; l < kNormLoads; ++l)
-                w[l] = kNT ? __builtin_nontemporal_load(q + l * kBlock) : q[l * kBlock];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int l = 0; l < kNormLoads; ++l) {
-#pragma unroll
-                for (int j = 0; j < E; ++j) {
-                    const double x = (double)(GV::at(w[l], j) * inv);
-                    acc[j & 1] = __builtin_fma(x, x, acc[j & 1]);
-                }
-            }
-        } else {  // a tensor's last tile: only the vectors (and elements) below its count
-#pragma unroll
-            for (int l = 0; l < kNormLoads; ++l) {
-                const uint32_t off = (uint32_t)(l * kBlock + threadIdx.x) * E;
-                const uint32_t nv = off < ch.count ? min(ch.count - off, (uint32_t)E) : 0u;
-                if (nv) {
-                    const R w = q[l * kBlock];
-#pragma unroll
-                    for (int j = 0; j < E; ++j) {
-                        const double x = (uint32_t)j < nv ? (double)(GV::at(w, j) * inv) : 0.0;
-                        acc[j & 1] = __builtin_fma(x, x, acc[j & 1]);
-                    }
-                }
-            }
-        }
-    }
-    const double b = block_sum(acc[0] + acc[1], lds);
-    if (threadIdx.x == 0) partials[blockIdx.x] = b;
-}
-
-// ------------------------------------------------------------------------------------
-// norm pass, part 2 (one block): combine the partials in index order (deterministic), then
-// decide found_inf / skip, the clip coefficient, the step count and the loss scale
+// the step's decisions: found_inf / skip, the clip coefficient, the step count, the loss scale
 // ------------------------------------------------------------------------------------
 struct FinalizeArgs {
     const double* partials;
@@ -345,23 +240,138 @@ __device__ __forceinline__ float bias_entry(const float* tab, uint32_t len, uint
     return (t >= 1 && t <= len) ? tab[2 * (t - 1) + j] : 1.0f;
 }
 
-__global__ __launch_bounds__(kBlock) void norm_finalize_kernel(FinalizeArgs a) {
-    __shared__ double lds[kBlock / 64];
+// the bias corrections of both outcomes: of t + 1 if the step applies, of t if it is skipped
+struct BiasPair {
+    float next1, next2, same1, same2;
+};
+__device__ __forceinline__ BiasPair load_bias(const FinalizeArgs& a, uint64_t t) {
+    if (!(a.count_t && a.want_bias)) return {1.0f, 1.0f, 1.0f, 1.0f};
+    return {bias_entry(a.bias_tab, a.bias_len, t + 1, 0), bias_entry(a.bias_tab, a.bias_len, t + 1, 1),
+            bias_entry(a.bias_tab, a.bias_len, t, 0), bias_entry(a.bias_tab, a.bias_len, t, 1)};
+}
+
+// what a step does, from the sum of squares of its unscaled gradients
+struct Decision {
+    double norm;
+    float inv, coef;
+    int32_t found, skip;
+};
+__device__ __forceinline__ float unscale_factor(const FinalizeArgs& a, float scale) {
+    return a.scaler_on ? (float)(1.0 / (double)scale) : 1.0f;
+}
+__device__ __forceinline__ Decision decide(const FinalizeArgs& a, float scale, double sumsq) {
+    Decision d;
+    d.inv = unscale_factor(a, scale);
+    d.norm = sqrt(sumsq);
+    d.found = !(sumsq <= 1.7976931348623157e308);  // inf or NaN
+    d.skip = a.scaler_on && d.found;
+    d.coef = 1.0f;
+    if (a.max_norm > 0.0) {
+        double cd = a.max_norm / (d.norm + 1e-6);
+        if (cd > 1.0) cd = 1.0;
+        d.coef = (float)cd;
+    }
+    return d;
+}
+
+// the step state after the step (one thread): s0 is the state before it
+__device__ __forceinline__ void write_state(const FinalizeArgs& a, const DevState& s0,
+                                            const BiasPair& b, double sumsq, const Decision& d) {
     DevState* st = a.st;
-    // Every load is issued before thread 0 decides: the first round of partials, then the
-    // whole step state (one 64-byte block, uniform, so scalar loads) and the bias corrections
-    // of both outcomes (t + 1 if the step applies, t if it is skipped), whose latency overlaps
-    // the partials' and their sum.  Read one after another, as the decisions need them, they
-    // were six dependent round trips on thread 0 after the sum.
-    // Partials: all loads of a round issued before the adds, each thread's order fixed
-    // (deterministic); with an index list (per-tensor sums), a round's indices load first.
-    // Loads past the end read the last entry and count as 0 in the adds (a branch or a select
-    // at each load made the compiler wait for it there).
+    st->sumsq = sumsq;
+    st->norm = d.norm;
+    if (a.probe) return;
+    st->found_inf = d.found;
+    st->skip = d.skip;
+    st->inv_scale = d.inv;
+    st->clip_coef = d.coef;
+    if (a.count_t) {
+        st->t = d.skip ? s0.t : s0.t + 1;
+        if (a.want_bias) {
+            st->bias1 = d.skip ? b.same1 : b.next1;
+            st->bias2 = d.skip ? b.same2 : b.next2;
+        }
+    }
+    if (a.scaler_on) {
+        if (a.defer_scale) {
+            st->pending = s0.pending | kPendingStep | (d.found ? kPendingInf : 0);
+        } else {
+            const ScaleUpdate u = next_scale(s0.scale, s0.growth_tracker, s0.pending, d.found,
+                                             a.growth_interval, a.growth_factor,
+                                             a.backoff_factor);
+            st->scale = u.scale;
+            st->growth_tracker = u.tracker;
+            st->pending = 0;
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------
+// the last block of a launch
+// ------------------------------------------------------------------------------------
+// A value that the launch's last block reads: stored and loaded as a relaxed atomic of device
+// scope, past the caches that other XCDs do not share.
+__device__ __forceinline__ void st_device(double* p, double x) {
+    __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double ld_device(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Tickets: kTicketGroups counters 128 B apart, which block b takes from counter b modulo
+// kTicketGroups, and one more that the last block of each group takes from.  One counter for a
+// whole launch made 2,048 blocks wait in line for the same word.  All are zero between
+// launches: the block that takes a counter's last ticket sets it back.
+constexpr uint32_t kTicketGroups = 32, kTicketPitch = 32;
+constexpr uint32_t kTicketWords = (kTicketGroups + 1) * kTicketPitch;
+__device__ __forceinline__ bool last_ticket(uint32_t* p, uint32_t of) {
+    const bool last =
+        __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == of - 1;
+    if (last) __hip_atomic_store(p, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return last;
+}
+
+// Whether this block is the launch's last to get here; every block of the launch calls it, with
+// all its lanes, after thread 0's st_device() stores, which the last block may then read with
+// ld_device().  Thread 0 waits until its stores have been acknowledged (device-scope stores
+// write through, so that is at memory) before it takes its ticket.  That wait takes the place of
+// a release fence: a device-scope fence per block also writes the XCD's L2 back and costs
+// ~50 ns per block, one block after another.
+// Measured (MLP AdamW with clipping, fp32): the step 9.0-9.5 us in two launches against 12.7 with
+// a launch of one block for the decisions; the norm kernel's tail takes about as long as that
+// launch did where the GPU is the bound (nanoGPT-char 53.7 against 53.6 us).
+__device__ __forceinline__ bool is_last_block(uint32_t* tickets, uint32_t* lds_flag) {
+    if (threadIdx.x == 0) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0);
+        asm volatile("" ::: "memory");
+        const uint32_t g = blockIdx.x % kTicketGroups;
+        const uint32_t size = (gridDim.x - g + kTicketGroups - 1) / kTicketGroups;
+        const uint32_t groups = min(gridDim.x, kTicketGroups);
+        *lds_flag = last_ticket(tickets + g * kTicketPitch, size) &&
+                    last_ticket(tickets + kTicketGroups * kTicketPitch, groups);
+    }
+    __syncthreads();
+    return *lds_flag != 0;
+}
+
+// One block of kBlock lanes combines the partials in index order (deterministic) and decides.
+// kLast: in the last block of the launch that stored the partials (see is_last_block).
+// Partials: all loads of a round issued before the adds, each thread's order fixed
+// (deterministic); with an index list (per-tensor sums), a round's indices load first.
+// Loads past the end read the last entry and count as 0 in the adds (a branch or a select
+// at each load made the compiler wait for it there).  s0 is the step state before the step,
+// which the caller loaded first; the bias corrections of both outcomes load beside the partials.
+template <bool kLast>
+__device__ __forceinline__ void finalize_block(const FinalizeArgs& a, const DevState& s0,
+                                               double* lds) {
     constexpr int kPer = 8;
     const uint32_t n = a.npartials;
-    double v[kPer];
-    auto load_round = [&](uint32_t base) {  // base < n
+    const BiasPair bias = load_bias(a, s0.t);
+    double s = 0.0;
+    for (uint32_t base = 0; base < n; base += kBlock * kPer) {
         uint32_t at[kPer];
+        double v[kPer];
 #pragma unroll
         for (int k = 0; k < kPer; ++k) at[k] = min(base + (uint32_t)k * kBlock + threadIdx.x, n - 1);
         if (a.idx) {
@@ -369,72 +379,142 @@ __global__ __launch_bounds__(kBlock) void norm_finalize_kernel(FinalizeArgs a) {
             for (int k = 0; k < kPer; ++k) at[k] = a.idx[at[k]];
         }
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) v[k] = a.partials[at[k]];
-    };
-    if (n) {
-        load_round(0);
-    } else {
-#pragma unroll
-        for (int k = 0; k < kPer; ++k) v[k] = 0.0;
-    }
-    const DevState s0 = *st;
-    float b1n = 1.0f, b2n = 1.0f, b1s = 1.0f, b2s = 1.0f;
-    if (a.count_t && a.want_bias) {
-        b1n = bias_entry(a.bias_tab, a.bias_len, s0.t + 1, 0);
-        b2n = bias_entry(a.bias_tab, a.bias_len, s0.t + 1, 1);
-        b1s = bias_entry(a.bias_tab, a.bias_len, s0.t, 0);
-        b2s = bias_entry(a.bias_tab, a.bias_len, s0.t, 1);
-    }
-    // keeps the compiler from moving the first round's adds (which wait for the partials)
-    // ahead of the state loads
-    __builtin_amdgcn_sched_barrier(0);
-    double s = 0.0;
-    for (uint32_t base = 0;;) {
+        for (int k = 0; k < kPer; ++k)
+            v[k] = kLast ? ld_device(a.partials + at[k]) : a.partials[at[k]];
 #pragma unroll
         for (int k = 0; k < kPer; ++k)
             s += base + (uint32_t)k * kBlock + threadIdx.x < n ? v[k] : 0.0;
-        base += kBlock * kPer;
-        if (base >= n) break;
-        load_round(base);
     }
     s = block_sum(s, lds);
-    if (threadIdx.x != 0) return;
+    if (threadIdx.x == 0) write_state(a, s0, bias, s, decide(a, s0.scale, s));
+}
 
-    const float inv = a.scaler_on ? (float)(1.0 / (double)s0.scale) : 1.0f;
-    const double norm = sqrt(s);
-    st->sumsq = s;
-    st->norm = norm;
-    if (a.probe) return;
-    const int found = !(s <= 1.7976931348623157e308);  // inf or NaN
-    const int skip = a.scaler_on && found;
-    float coef = 1.0f;
-    if (a.max_norm > 0.0) {
-        double cd = a.max_norm / (norm + 1e-6);
-        if (cd > 1.0) cd = 1.0;
-        coef = (float)cd;
+// the decisions alone, in a launch of one block: without a norm pass (step counting), or over
+// per-tensor sums
+__global__ __launch_bounds__(kBlock) void norm_finalize_kernel(FinalizeArgs a) {
+    __shared__ double lds[kBlock / 64];
+    const DevState s0 = *a.st;
+    finalize_block<false>(a, s0, lds);
+}
+
+// ------------------------------------------------------------------------------------
+// norm pass: per-block partial sums of squares of the unscaled gradients, and the decisions
+// ------------------------------------------------------------------------------------
+// 16-byte loads: 8 bf16 or 4 fp32 gradients per lane
+template <typename GradT>
+struct GradVec;
+template <>
+struct GradVec<uint16_t> {
+    static constexpr int kElems = 8;
+    typedef uint32_t raw __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ float at(const raw& w, int j) {
+        return (j & 1) ? bf16_hi(w[j >> 1]) : bf16_lo(w[j >> 1]);
     }
-    st->found_inf = found;
-    st->skip = skip;
-    st->inv_scale = inv;
-    st->clip_coef = coef;
-    if (a.count_t) {
-        st->t = skip ? s0.t : s0.t + 1;
-        if (a.want_bias) {
-            st->bias1 = skip ? b1s : b1n;
-            st->bias2 = skip ? b2s : b2n;
+    // element j of a vector that starts as zeros
+    static __device__ __forceinline__ void put(raw& w, int j, uint16_t h) {
+        w[j >> 1] |= (j & 1) ? ((uint32_t)h << 16) : (uint32_t)h;
+    }
+};
+template <>
+struct GradVec<float> {
+    static constexpr int kElems = 4;
+    typedef f32x4 raw;
+    static __device__ __forceinline__ float at(const raw& w, int j) { return w[j]; }
+    static __device__ __forceinline__ void put(raw& w, int j, float x) { w[j] = x; }
+};
+
+// Norm tiles: kNormLoads 16-byte loads per lane, so a tile is 16 KiB of gradients (8192 bf16
+// or 4096 fp32); the pass has its own tile table (same tensors, bigger pieces than the update's
+// chunks) so each descriptor fetch is amortised over 4 loads per lane.
+constexpr int kNormLoads = 4;
+template <typename GradT>
+constexpr uint32_t norm_tile_elems() {
+    return (uint32_t)(kBlock * kNormLoads * 16 / sizeof(GradT));
+}
+
+// Grid-stride over the norm tiles t0 .. t1-1, one partial per block.  A whole tile (every tile
+// but a tensor's last) is four unconditional 16-byte loads per lane, all issued before the
+// arithmetic (the scheduling barrier keeps the compiler from interleaving them with it, which
+// left one or two loads in flight: 6.0-6.3 TB/s against 6.7-6.9 at GPT-2 774M / 1558M).
+// kNT selects non-temporal loads.  The host runs the pass as two launches: non-temporal over
+// all but the last kCachedGradBytes of gradients, then cached loads over those, which the
+// update, walking the chunks in reverse, reads first and so finds in the 256 MB Infinity
+// Cache (measured on GPT-2 124M: update 531 us after this pass vs 559 us alone; at 774M and
+// 1558M fp32 the split pass runs 232 and 931 us against 246-260 and 978-1030 us with cached
+// loads throughout, the update unchanged).  Each block writes one partial, and with kDecide the
+// launch's last block combines all of them (an earlier launch's included) and decides.  Squares
+// of fp32 values are exact in fp64, and any inf/NaN gradient makes the sum non-finite.
+template <typename GradT, bool kNT, bool kDecide>
+__global__ __launch_bounds__(kBlock) void norm_partials_kernel(const GradT* __restrict__ g,
+                                                               const Chunk* __restrict__ tiles,
+                                                               uint32_t t0, uint32_t t1,
+                                                               const DevState* __restrict__ st,
+                                                               int32_t scaler_on,
+                                                               double* __restrict__ partials,
+                                                               FinalizeArgs fin,
+                                                               uint32_t* __restrict__ tickets) {
+    typedef GradVec<GradT> GV;
+    typedef typename GV::raw R;
+    constexpr int E = GV::kElems;
+    constexpr uint32_t kTile = norm_tile_elems<GradT>();
+    __shared__ double lds[kBlock / 64];
+    // The first tile's descriptor and the step state load together, ahead of the arithmetic on
+    // the scale, and each further descriptor beside the tile before it: one round trip less
+    // before each tile's data than with the loads where their values are used.
+    uint32_t c = t0 + blockIdx.x;
+    Chunk ch = load_chunk(tiles, c < t1 ? c : t0);
+    const DevState s0 = *st;  // whole, since any block may be the launch's last
+    // both are here from this point on (left to itself, the compiler loads the descriptor after
+    // the division)
+    asm volatile("" ::"s"(ch.count), "s"(s0.scale) : "memory");
+    const float inv = scaler_on ? (float)(1.0 / (double)s0.scale) : 1.0f;
+    // two accumulators (element j of a vector goes to acc[j & 1]): a fixed order, so the
+    // sum stays deterministic, with half the dependent-add chain.  The square of an fp32 value
+    // is exact in fp64, so fma(x, x, acc) rounds exactly as acc + x*x does (one rounding, of
+    // the add) with one instruction instead of two.
+    double acc[2] = {0.0, 0.0};
+    for (; c < t1; c += gridDim.x) {
+        const R* q = reinterpret_cast<const R*>(g + ch.begin) + threadIdx.x;
+        const uint32_t count = ch.count;
+        const uint32_t next = c + gridDim.x;  // (below 2^24 + 2^17 tiles and blocks: no wrap)
+        ch = load_chunk(tiles, next < t1 ? next : c);
+        if (count == kTile) {
+            R w[kNormLoads];
+#pragma unroll
+            for (int l = 0; l < kNormLoads; ++l)
+                w[l] = kNT ? __builtin_nontemporal_load(q + l * kBlock) : q[l * kBlock];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int l = 0; l < kNormLoads; ++l) {
+#pragma unroll
+                for (int j = 0; j < E; ++j) {
+                    const double x = (double)(GV::at(w[l], j) * inv);
+                    acc[j & 1] = __builtin_fma(x, x, acc[j & 1]);
+                }
+            }
+        } else {  // a tensor's last tile: only the vectors (and elements) below its count
+#pragma unroll
+            for (int l = 0; l < kNormLoads; ++l) {
+                const uint32_t off = (uint32_t)(l * kBlock + threadIdx.x) * E;
+                const uint32_t nv = off < count ? min(count - off, (uint32_t)E) : 0u;
+                if (nv) {
+                    const R w = q[l * kBlock];
+#pragma unroll
+                    for (int j = 0; j < E; ++j) {
+                        const double x = (uint32_t)j < nv ? (double)(GV::at(w, j) * inv) : 0.0;
+                        acc[j & 1] = __builtin_fma(x, x, acc[j & 1]);
+                    }
+                }
+            }
         }
     }
-    if (a.scaler_on) {
-        if (a.defer_scale) {
-            st->pending = s0.pending | kPendingStep | (found ? kPendingInf : 0);
-        } else {
-            const ScaleUpdate u = next_scale(s0.scale, s0.growth_tracker, s0.pending, found,
-                                             a.growth_interval, a.growth_factor,
-                                             a.backoff_factor);
-            st->scale = u.scale;
-            st->growth_tracker = u.tracker;
-            st->pending = 0;
-        }
+    const double b = block_sum(acc[0] + acc[1], lds);
+    if constexpr (kDecide) {
+        __shared__ uint32_t last;
+        if (threadIdx.x == 0) st_device(partials + blockIdx.x, b);
+        if (is_last_block(tickets, &last)) finalize_block<true>(fin, s0, lds);
+    } else {
+        if (threadIdx.x == 0) partials[blockIdx.x] = b;
     }
 }
 
@@ -513,16 +593,20 @@ __device__ __forceinline__ double tile_from_waves(const double* __restrict__ w, 
 // partials of its tiles, from kWaves x tile_base[tensor]), if it has any pending: each tile
 // from its waves, then the tiles in sum_tiles' order, so the tensor's sum equals what
 // ttp_grad_sumsq_tensors gives for the same gradients.  One launch per step instead of one
-// per accumulate.
+// per accumulate; its last block combines the sums of all stepped tensors and decides.
 __global__ __launch_bounds__(kBlock) void combine_pending_sums_kernel(
     const double* __restrict__ acc_waves, const uint32_t* __restrict__ tile_base,
     const uint32_t* __restrict__ tile_start, const uint32_t* __restrict__ tensor_ids,
-    uint32_t* __restrict__ pending, double* __restrict__ sums) {
+    uint32_t* __restrict__ pending, double* __restrict__ sums, FinalizeArgs fin,
+    uint32_t* __restrict__ tickets) {
     __shared__ double lds[kBlock / 64];
+    __shared__ uint32_t last;
+    const DevState s0 = *fin.st;  // any block may be the last
+    asm volatile("" ::: "memory");
     const uint32_t t = blockIdx.x, i = tensor_ids[t];
-    if (!pending[i]) return;  // uniform over the block
     const double* w = acc_waves + (uint64_t)tile_base[i] * kWaves;
-    const uint32_t e = tile_start[t + 1] - tile_start[t];
+    // nothing pending (uniform over the block): the sum is there already
+    const uint32_t e = pending[i] ? tile_start[t + 1] - tile_start[t] : 0u;
     // sum_tiles' order, rounds and unconditional loads, over tile values formed from the wave
     // partials
     constexpr int kPer = kSumRound;
@@ -535,11 +619,14 @@ __global__ __launch_bounds__(kBlock) void combine_pending_sums_kernel(
 #pragma unroll
         for (int k = 0; k < kPer; ++k) s += base + (uint32_t)k * kBlock + threadIdx.x < e ? v[k] : 0.0;
     }
-    s = block_sum(s, lds);
-    if (threadIdx.x == 0) {
-        sums[i] = s;
-        pending[i] = 0u;
+    if (e) {
+        s = block_sum(s, lds);
+        if (threadIdx.x == 0) {
+            st_device(sums + i, s);
+            pending[i] = 0u;
+        }
     }
+    if (is_last_block(tickets, &last)) finalize_block<true>(fin, s0, lds);
 }
 
 // ------------------------------------------------------------------------------------

@@ -174,6 +174,7 @@ struct ttp_ctx {
     DevState* st = nullptr;
     double* partials = nullptr;
     uint32_t partials_cap = 0;
+    uint32_t* tickets = nullptr;  // the last block of a launch (ttp::is_last_block)
 
     uint32_t norm_grid_cap = 0;  // blocks of the norm pass (one partial each)
     uint32_t upd_lds = 0;        // dynamic LDS per update block (caps blocks per CU)
@@ -760,23 +761,26 @@ NormSplit norm_split(const ttp_ctx* c, uint32_t n) {
     return s;
 }
 
+// the norm pass; its last launch's last block decides (fin)
 template <typename GradT>
 void launch_norm_pass(ttp_ctx* c, const WorkTables* w, const NormSplit& ns, int32_t scaler_on,
-                      double* partials) {
+                      double* partials, const ttp::FinalizeArgs& fin) {
     const GradT* g = (const GradT*)c->grad;
     const DevState* st = c->st;
     if (ns.g_nt)
-        hipLaunchKernelGGL((ttp::norm_partials_kernel<GradT, true>), dim3(ns.g_nt),
+        hipLaunchKernelGGL((ttp::norm_partials_kernel<GradT, true, false>), dim3(ns.g_nt),
                            dim3(ttp::kBlock), 0, c->stream, g, w->tiles, 0u, ns.split, st,
-                           scaler_on, partials);
-    hipLaunchKernelGGL((ttp::norm_partials_kernel<GradT, false>), dim3(ns.g_cached),
+                           scaler_on, partials, fin, (uint32_t*)nullptr);
+    hipLaunchKernelGGL((ttp::norm_partials_kernel<GradT, false, true>), dim3(ns.g_cached),
                        dim3(ttp::kBlock), 0, c->stream, g, w->tiles, ns.split, w->n_tiles, st,
-                       scaler_on, partials + ns.g_nt);
+                       scaler_on, partials + ns.g_nt, fin, c->tickets);
 }
 
-// Step prologue on the device: the norm pass (partials, when `run_norm`) and the one-block
-// finalize (norm, found_inf / skip, clip coefficient, loss scale, and the step count with its
-// bias corrections when `count_t`); `probe` only computes the norm.
+// Step prologue on the device: the norm pass (when `run_norm`) and the decisions (norm,
+// found_inf / skip, clip coefficient, loss scale, and the step count with its bias corrections
+// when `count_t`), taken by the last block of the last launch before the update: the norm
+// pass's, or that of the pending sums' combination; a launch of its own remains where neither
+// runs.  `probe` only computes the norm.
 // `partials` (null: the context's own) holds one partial per norm-pass block; a caller-given
 // array (the no-allocation step's) also turns the per-launch timing events off.
 int launch_prologue(ttp_ctx* c, const WorkTables* w, bool run_norm, double max_norm, bool probe,
@@ -786,28 +790,10 @@ int launch_prologue(ttp_ctx* c, const WorkTables* w, bool run_norm, double max_n
     const int32_t scaler_on = c->scaler.enabled ? 1 : 0;
     TimedLaunch tl(c, TTP_KERNEL_NORM, partials == nullptr);
     if (!partials) partials = c->partials;
-    if (run_norm && !from_sums) {
-        clear_hip_error();
-        if (bf16_grads(c))
-            launch_norm_pass<uint16_t>(c, w, ns, scaler_on, partials);
-        else
-            launch_norm_pass<float>(c, w, ns, scaler_on, partials);
-        HIP_TRY(hipGetLastError());
-    }
     ttp::FinalizeArgs a{};
     a.partials = partials;
     a.npartials = run_norm ? ns.partials() : 0;
     if (run_norm && from_sums) {  // the step's tensors' sums, in tensor order
-        // tile sums that accumulates with their sums left pending: combined first (a captured
-        // step always launches this, since its replays may find them pending)
-        if (w->n_tensors && (c->capturing || c->acc_sums_used)) {
-            clear_hip_error();
-            hipLaunchKernelGGL(ttp::combine_pending_sums_kernel, dim3(w->n_tensors),
-                               dim3(ttp::kBlock), 0, c->stream, (const double*)c->acc_tiles,
-                               (const uint32_t*)c->tile_base, (const uint32_t*)w->tile_start,
-                               (const uint32_t*)w->tensor_ids, c->tsum_pending, c->tsum);
-            HIP_TRY(hipGetLastError());
-        }
         a.partials = c->tsum;
         a.idx = w->tensor_ids;
         a.npartials = w->n_tensors;
@@ -825,7 +811,23 @@ int launch_prologue(ttp_ctx* c, const WorkTables* w, bool run_norm, double max_n
     a.want_bias = want_bias ? 1 : 0;
     a.st = c->st;
     clear_hip_error();
-    hipLaunchKernelGGL(ttp::norm_finalize_kernel, dim3(1), dim3(ttp::kBlock), 0, c->stream, a);
+    if (run_norm && !from_sums) {
+        if (bf16_grads(c))
+            launch_norm_pass<uint16_t>(c, w, ns, scaler_on, partials, a);
+        else
+            launch_norm_pass<float>(c, w, ns, scaler_on, partials, a);
+    } else if (run_norm && w->n_tensors && (c->capturing || c->acc_sums_used)) {
+        // tile sums that accumulates with their sums left pending: combined first (a captured
+        // step always launches this, since its replays may find them pending)
+        hipLaunchKernelGGL(ttp::combine_pending_sums_kernel, dim3(w->n_tensors),
+                           dim3(ttp::kBlock), 0, c->stream, (const double*)c->acc_tiles,
+                           (const uint32_t*)c->tile_base, (const uint32_t*)w->tile_start,
+                           (const uint32_t*)w->tensor_ids, c->tsum_pending, c->tsum, a,
+                           c->tickets);
+    } else {
+        hipLaunchKernelGGL(ttp::norm_finalize_kernel, dim3(1), dim3(ttp::kBlock), 0, c->stream,
+                           a);
+    }
     HIP_TRY(hipGetLastError());
     tl.done();
     return TTP_OK;
@@ -1106,7 +1108,7 @@ void release(ttp_ctx* c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : {(void*)c->grad, (void*)c->records, (void*)c->momentum, (void*)c->mom_init,
-                    (void*)c->st, (void*)c->partials, c->staging, (void*)c->tsum,
+                    (void*)c->st, (void*)c->partials, (void*)c->tickets, c->staging, (void*)c->tsum,
                     (void*)c->tile_sums, (void*)c->acc_tiles, (void*)c->tile_base,
                     (void*)c->tsum_pending})
         if (p) (void)hipFree(p);
@@ -1253,6 +1255,7 @@ int ttp_create(int device, const ttp_tensor_desc* descs, uint32_t n, int mode, t
     if ((rc = alloc_zero(c, (void**)&c->st, sizeof(DevState)))) return bail(rc);
     c->partials_cap = 2 * c->norm_grid_cap;  // the norm pass's two launches (NormSplit)
     if ((rc = alloc_zero(c, (void**)&c->partials, (uint64_t)c->partials_cap * 8))) return bail(rc);
+    if ((rc = alloc_zero(c, (void**)&c->tickets, ttp::kTicketWords * 4))) return bail(rc);
     if ((rc = alloc_zero(c, (void**)&c->tsum, std::max<uint64_t>(n, 1) * 8))) return bail(rc);
     c->tsum_fresh.assign(n, 0);
     // the tile sums of accumulates with their sums: 32 B per 16 KiB of gradients
@@ -2125,14 +2128,17 @@ int ttp_grad_sumsq_tensors(ttp_ctx* c, const uint32_t* indices, uint32_t n) {
         const int32_t scaler_on = c->scaler.enabled ? 1 : 0;
         clear_hip_error();
         if (bf16_grads(c))
-            hipLaunchKernelGGL((ttp::norm_partials_kernel<uint16_t, false>), dim3(w->n_tiles),
-                               dim3(ttp::kBlock), 0, c->stream, (const uint16_t*)c->grad,
-                               w->tiles, 0u, w->n_tiles, (const DevState*)c->st, scaler_on,
-                               c->tile_sums);
+            hipLaunchKernelGGL((ttp::norm_partials_kernel<uint16_t, false, false>),
+                               dim3(w->n_tiles), dim3(ttp::kBlock), 0, c->stream,
+                               (const uint16_t*)c->grad, w->tiles, 0u, w->n_tiles,
+                               (const DevState*)c->st, scaler_on, c->tile_sums,
+                               ttp::FinalizeArgs{}, (uint32_t*)nullptr);
         else
-            hipLaunchKernelGGL((ttp::norm_partials_kernel<float, false>), dim3(w->n_tiles),
-                               dim3(ttp::kBlock), 0, c->stream, (const float*)c->grad, w->tiles,
-                               0u, w->n_tiles, (const DevState*)c->st, scaler_on, c->tile_sums);
+            hipLaunchKernelGGL((ttp::norm_partials_kernel<float, false, false>),
+                               dim3(w->n_tiles), dim3(ttp::kBlock), 0, c->stream,
+                               (const float*)c->grad, w->tiles, 0u, w->n_tiles,
+                               (const DevState*)c->st, scaler_on, c->tile_sums,
+                               ttp::FinalizeArgs{}, (uint32_t*)nullptr);
         HIP_TRY(hipGetLastError());
         clear_hip_error();
         hipLaunchKernelGGL(ttp::tensor_sums_kernel, dim3(w->n_tensors), dim3(ttp::kBlock), 0,
