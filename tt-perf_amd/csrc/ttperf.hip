@@ -776,6 +776,47 @@ void launch_norm_pass(ttp_ctx* c, const WorkTables* w, const NormSplit& ns, int3
                        scaler_on, partials + ns.g_nt, fin, c->tickets);
 }
 
+// The decisions' arguments, with no partials yet.
+ttp::FinalizeArgs finalize_args(const ttp_ctx* c, bool run_norm, double max_norm, bool probe,
+                                bool want_bias, bool count_t, bool defer_scale) {
+    ttp::FinalizeArgs a{};
+    a.scaler_on = run_norm && c->scaler.enabled ? 1 : 0;
+    a.defer_scale = defer_scale ? 1 : 0;
+    a.count_t = count_t ? 1 : 0;
+    a.probe = probe ? 1 : 0;
+    a.growth_interval = c->scaler.growth_interval;
+    a.growth_factor = c->scaler.growth_factor;
+    a.backoff_factor = c->scaler.backoff_factor;
+    a.max_norm = run_norm ? max_norm : 0.0;
+    a.bias_tab = c->bias_tab;
+    a.bias_len = c->bias_len;
+    a.want_bias = want_bias ? 1 : 0;
+    a.st = c->st;
+    return a;
+}
+
+// Whether a step that needs the norm or counts on the device (else it is one launch anyway) runs
+// as one launch (see ttp::adam_small_kernel and its likes).  Every block reads all gradients, so
+// the set must be small: at most kSmallElems elements in kSmallTiles norm tiles.  AdamW steps
+// with clipping from Python, us in one / two launches: 10,000 parameters 6.1 / 9.3, 32,768
+// 7.5-7.7 / 8.7-9.4, 49,152 8.7-9.3 / 8.7-9.4, 65,536 9.5-10.3 / 8.6-9.3 (fp32 and mixed); 15
+// tensors of 300 elements 6.8 / 10.0, 60 of them 10.5 / 13.1-13.6.  Per-tensor sums take the
+// norm from elsewhere, and per-kernel timing times the norm pass and the update apart.
+constexpr uint64_t kSmallElems = 32768;
+bool one_launch_step(const ttp_ctx* c, const WorkTables* w, bool prologue, bool from_sums) {
+    return prologue && !from_sums && !c->timing && w->n_chunks &&
+           w->n_tiles <= ttp::kSmallTiles && w->elems <= kSmallElems;
+}
+ttp::SmallArgs small_args(const ttp_ctx* c, const WorkTables* w, bool run_norm,
+                          const ttp::FinalizeArgs& fin) {
+    ttp::SmallArgs s{};
+    s.fin = fin;
+    s.tiles = w->tiles;
+    s.ntiles = run_norm ? w->n_tiles : 0;
+    s.tickets = c->tickets;
+    return s;
+}
+
 // Step prologue on the device: the norm pass (when `run_norm`) and the decisions (norm,
 // found_inf / skip, clip coefficient, loss scale, and the step count with its bias corrections
 // when `count_t`), taken by the last block of the last launch before the update: the norm
@@ -790,7 +831,8 @@ int launch_prologue(ttp_ctx* c, const WorkTables* w, bool run_norm, double max_n
     const int32_t scaler_on = c->scaler.enabled ? 1 : 0;
     TimedLaunch tl(c, TTP_KERNEL_NORM, partials == nullptr);
     if (!partials) partials = c->partials;
-    ttp::FinalizeArgs a{};
+    ttp::FinalizeArgs a = finalize_args(c, run_norm, max_norm, probe, want_bias, count_t,
+                                        defer_scale);
     a.partials = partials;
     a.npartials = run_norm ? ns.partials() : 0;
     if (run_norm && from_sums) {  // the step's tensors' sums, in tensor order
@@ -798,18 +840,6 @@ int launch_prologue(ttp_ctx* c, const WorkTables* w, bool run_norm, double max_n
         a.idx = w->tensor_ids;
         a.npartials = w->n_tensors;
     }
-    a.scaler_on = run_norm ? scaler_on : 0;
-    a.defer_scale = defer_scale ? 1 : 0;
-    a.count_t = count_t ? 1 : 0;
-    a.probe = probe ? 1 : 0;
-    a.growth_interval = c->scaler.growth_interval;
-    a.growth_factor = c->scaler.growth_factor;
-    a.backoff_factor = c->scaler.backoff_factor;
-    a.max_norm = run_norm ? max_norm : 0.0;
-    a.bias_tab = c->bias_tab;
-    a.bias_len = c->bias_len;
-    a.want_bias = want_bias ? 1 : 0;
-    a.st = c->st;
     clear_hip_error();
     if (run_norm && !from_sums) {
         if (bf16_grads(c))
@@ -1834,7 +1864,8 @@ static int adam_step_impl(ttp_ctx* c, const ttp_adam_hparams* hp, const uint32_t
     // m and v last, once nothing above can refuse the step: in the SGD layout this moves the
     // master into new records, which a refused call must not do
     if ((rc = ensure_adam_state(c))) return rc;
-    if ((need_norm || devt) &&
+    const bool small = one_launch_step(c, w, need_norm || devt, from_sums);
+    if ((need_norm || devt) && !small &&
         (rc = launch_prologue(c, w, need_norm, hp->max_grad_norm, false, devt, devt, from_sums,
                               defer, scratch_partials)))
         return rc;
@@ -1871,7 +1902,19 @@ static int adam_step_impl(ttp_ctx* c, const ttp_adam_hparams* hp, const uint32_t
         ttp::AdamArgs al = a;
         al.st = c->st;  // the lane forms read the device state unconditionally
         clear_hip_error();
-        if (grads_cached(c, w) && c->mode == TTP_MODE_MIXED)
+        if (small) {
+            const ttp::SmallArgs s =
+                small_args(c, w, need_norm, finalize_args(c, need_norm, hp->max_grad_norm, false,
+                                                          devt, devt, defer));
+            if (c->mode == TTP_MODE_MIXED)
+                hipLaunchKernelGGL((ttp::adam_small_kernel<uint16_t, true>), dim3(n),
+                                   dim3(ttp::kSmallBlock), 0, c->stream, g16, c->records,
+                                   (float*)nullptr, p16, a, s);
+            else
+                hipLaunchKernelGGL((ttp::adam_small_kernel<float, false>), dim3(n),
+                                   dim3(ttp::kSmallBlock), 0, c->stream, g32, c->records,
+                                   c->master, (uint16_t*)nullptr, a, s);
+        } else if (grads_cached(c, w) && c->mode == TTP_MODE_MIXED)
             launch_lanes(c,
                          (uint64_t)n * ttp::lane_parts<kLaneAdamMixedCached, kLanesAdamMixedCached,
                                                        kItAdamMixedCached>(),
@@ -1947,11 +1990,20 @@ static int sgd_step_impl(ttp_ctx* c, const ttp_sgd_hparams* hp, const uint32_t* 
     // the momentum buffer once nothing above can refuse the step (a refused call changes
     // nothing, not even what a checkpoint would hold)
     if (mom && (rc = ensure_momentum(c))) return rc;
-    if ((need_norm || devt) &&
+    const bool small = one_launch_step(c, w, need_norm || devt, from_sums);
+    if ((need_norm || devt) && !small &&
         (rc = launch_prologue(c, w, need_norm, hp->max_grad_norm, false, false, devt, from_sums,
                               defer)))
         return rc;
     if (!devt) c->host_t += 1;
+    // With momentum, the stepped tensors hold a momentum buffer after the step (torch: state
+    // created on first use).  They are marked where the host does not know them marked: with
+    // loss scaling the device decides, since the step may be skipped, and once captured the
+    // marking is part of every replay.
+    bool mark = mom && (scaler || devt);
+    if (mom)
+        for (uint32_t i : active)
+            if (!c->host_mom_init[i]) mark = true;
 
     ttp::SgdArgs a{};
     a.chunks = chunks;
@@ -1981,7 +2033,31 @@ static int sgd_step_impl(ttp_ctx* c, const ttp_sgd_hparams* hp, const uint32_t* 
         hipLaunchKernelGGL((ttp::sgd_lane_kernel<GT, MIXED, MS, E, LN, IT>), g, dim3(LN), 0,  \
                            c->stream, G, c->master, c->momentum, P16, al, p0);                \
     })
-        if (c->mode == TTP_MODE_BF16)
+        if (small) {
+            ttp::SmallArgs s =
+                small_args(c, w, need_norm, finalize_args(c, need_norm, hp->max_grad_norm, false,
+                                                          false, devt, defer));
+            if (mark) {
+                s.mom_init = c->mom_init;
+                s.mom_ids = w->tensor_ids;
+                s.n_mom = w->n_tensors;
+            }
+            const dim3 sblock(ttp::kSmallBlock);
+            if (c->mode == TTP_MODE_BF16)
+                hipLaunchKernelGGL(ttp::sgd_bf16_small_kernel, dim3(n), sblock, 0, c->stream, g16,
+                                   p16, a, s);
+            else if (c->mode == TTP_MODE_MIXED && c->sgd_layout)
+                hipLaunchKernelGGL((ttp::sgd_small_kernel<uint16_t, true, ttp::kRec>), dim3(n),
+                                   sblock, 0, c->stream, g16, c->master, c->momentum, p16, a, s);
+            else if (c->mode == TTP_MODE_MIXED)
+                hipLaunchKernelGGL((ttp::sgd_small_kernel<uint16_t, true, ttp::kStrideMixed>),
+                                   dim3(n), sblock, 0, c->stream, g16, c->master, c->momentum,
+                                   p16, a, s);
+            else
+                hipLaunchKernelGGL((ttp::sgd_small_kernel<float, false, ttp::kRec>), dim3(n),
+                                   sblock, 0, c->stream, g32, c->master, c->momentum,
+                                   (uint16_t*)nullptr, a, s);
+        } else if (c->mode == TTP_MODE_BF16)
             launch_lanes(c, (uint64_t)n * ttp::lane_parts<kLaneSgdBf16, kLanesSgdBf16, kItSgdBf16>(),
                          kLanesSgdBf16, [&](dim3 g, uint64_t p0) {
                 hipLaunchKernelGGL((ttp::sgd_bf16_lane_kernel<kLaneSgdBf16, kLanesSgdBf16,
@@ -2013,25 +2089,17 @@ static int sgd_step_impl(ttp_ctx* c, const ttp_sgd_hparams* hp, const uint32_t* 
 #undef TTP_SGD_LANES
         HIP_TRY(hipGetLastError());
         tl.done();
-        if (mom) {
-            // the stepped tensors now hold a momentum buffer (torch: state created on first
-            // use); with loss scaling the device decides, since the step may be skipped, and
-            // once captured the marking is part of every replay
-            bool needed = scaler || devt;
-            for (uint32_t i : active)
-                if (!c->host_mom_init[i]) needed = true;
-            if (needed) {
-                const uint32_t g =
-                    std::max<uint32_t>(1, std::min<uint32_t>((n + ttp::kBlock - 1) / ttp::kBlock, 1024));
-                clear_hip_error();
-                hipLaunchKernelGGL(ttp::mark_mom_init_kernel, dim3(g), dim3(ttp::kBlock), 0,
-                                   c->stream, chunks, n, c->mom_init, (const DevState*)c->st,
-                                   scaler ? 1 : 0);
-                HIP_TRY(hipGetLastError());
-            }
-            if (!scaler && !devt)
-                for (uint32_t i : active) c->host_mom_init[i] = 1;
+        if (mark && !small) {
+            const uint32_t g =
+                std::max<uint32_t>(1, std::min<uint32_t>((n + ttp::kBlock - 1) / ttp::kBlock, 1024));
+            clear_hip_error();
+            hipLaunchKernelGGL(ttp::mark_mom_init_kernel, dim3(g), dim3(ttp::kBlock), 0,
+                               c->stream, chunks, n, c->mom_init, (const DevState*)c->st,
+                               scaler ? 1 : 0);
+            HIP_TRY(hipGetLastError());
         }
+        if (mom && !scaler && !devt)
+            for (uint32_t i : active) c->host_mom_init[i] = 1;
     }
     consume_sums(c, active, scaler && !defer);
     if (report) return fill_report(c, need_norm, report);
