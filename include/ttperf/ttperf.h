@@ -250,6 +250,8 @@ int ttp_destroy(ttp_ctx* ctx);
 int ttp_set_stream(ttp_ctx* ctx, void* hip_stream);
 /* Back to the context's own (non-blocking) stream. */
 int ttp_reset_stream(ttp_ctx* ctx);
+/* The stream the context's work is ordered on (the caller's, or the context's own). */
+int ttp_get_stream(const ttp_ctx* ctx, void** hip_stream);
 int ttp_sync(ttp_ctx* ctx);
 
 /* ---- layout ------------------------------------------------------------------------- */

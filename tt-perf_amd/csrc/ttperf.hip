@@ -897,9 +897,19 @@ int fill_report(ttp_ctx* c, bool norm_ran, ttp_step_report* r) {
 // A caller's buffer that the GPU reads or writes directly (TTP_DEVICE transfers, device
 // gradient sources): [p, p + bytes) must be device (or managed) memory of this context's
 // device, inside one allocation.  A host pointer, another device's memory or a short buffer
-// is refused here, before any launch or copy touches it.
-int check_device_buffer(const ttp_ctx* c, const void* p, uint64_t bytes, const char* what) {
+// is refused here, before any launch or copy touches it.  `seen`, for a call that checks several
+// buffers: the allocation the last of them was found in, which answers for the next one there
+// (a bucket's gradients are mostly slices of one allocation; the runtime's two queries take
+// about a microsecond per buffer).
+struct SeenAlloc {
+    uintptr_t lo = 0, end = 0;
+};
+int check_device_buffer(const ttp_ctx* c, const void* p, uint64_t bytes, const char* what,
+                        SeenAlloc* seen = nullptr) {
     if (!bytes) return TTP_OK;
+    if (seen && (uintptr_t)p >= seen->lo && (uintptr_t)p < seen->end &&
+        bytes <= seen->end - (uintptr_t)p)
+        return TTP_OK;
     hipPointerAttribute_t at{};
     if (hipPointerGetAttributes(&at, p) != hipSuccess) {
         clear_hip_error();
@@ -924,6 +934,7 @@ int check_device_buffer(const ttp_ctx* c, const void* p, uint64_t bytes, const c
         return fail(TTP_ERR_RANGE, std::string(what) + ": " + std::to_string(bytes) +
                                        " bytes do not fit its allocation (" +
                                        std::to_string(end - lo) + " bytes from the pointer on)");
+    if (seen) *seen = {(uintptr_t)base, end};
     return TTP_OK;
 }
 
@@ -1361,6 +1372,14 @@ int ttp_reset_stream(ttp_ctx* c) {
     return TTP_OK;
 }
 
+int ttp_get_stream(const ttp_ctx* c, void** stream) {
+    int rc = check_ctx(c);
+    if (rc) return rc;
+    if (!stream) return fail(TTP_ERR_INVALID, "null output");
+    *stream = c->stream;
+    return TTP_OK;
+}
+
 int ttp_sync(ttp_ctx* c) {
     int rc = check_ctx(c);
     if (rc) return rc;
@@ -1741,6 +1760,7 @@ int ttp_accumulate_grad_multi(ttp_ctx* c, const uint32_t* indices, const void* c
     ttp::MultiAccArgs a{};
     uint64_t tiles = 0;
     bool vec = true;
+    SeenAlloc seen_alloc;
     // every check first: a refused call changes nothing
     for (uint32_t k = 0; k < n; ++k) {
         const uint32_t i = indices[k];
@@ -1758,7 +1778,8 @@ int ttp_accumulate_grad_multi(ttp_ctx* c, const uint32_t* indices, const void* c
         const TensorRec& t = c->tensors[i];
         if (!t.numel) continue;
         if (!srcs[k]) return fail(TTP_ERR_INVALID, "null source for tensor " + std::to_string(i));
-        if ((rc = check_device_buffer(c, srcs[k], t.numel * sbytes, "an incoming gradient")))
+        if ((rc = check_device_buffer(c, srcs[k], t.numel * sbytes, "an incoming gradient",
+                                      &seen_alloc)))
             return rc;
         vec = vec && ((uintptr_t)srcs[k] & 15u) == 0;
         tiles += (t.numel + tile - 1) / tile;

@@ -67,6 +67,7 @@ SIGNATURES = {
     "ttp_destroy": (C.c_int, [_P]),
     "ttp_set_stream": (C.c_int, [_P, _P]),
     "ttp_reset_stream": (C.c_int, [_P]),
+    "ttp_get_stream": (C.c_int, [_P, C.POINTER(_P)]),
     "ttp_sync": (C.c_int, [_P]),
     "ttp_num_tensors": (C.c_int, [_P, C.POINTER(C.c_uint32)]),
     "ttp_mode": (C.c_int, [_P, C.POINTER(C.c_int)]),

@@ -22,6 +22,8 @@ when clipping or loss scaling), instead of ~15 elementwise programs per tensor.
 """
 from __future__ import annotations
 
+import ctypes as C
+import operator
 import weakref
 
 from . import _lib as L
@@ -37,15 +39,31 @@ def _group_by_store(params, what):
     return list(groups.values())
 
 
+def _with_indices(groups):
+    """[(store, members, their sorted indices as the ABI takes them)]"""
+    out = []
+    for store, members in groups:
+        idx = sorted({p.index for p in members})
+        out.append((store, members, (C.c_uint32 * len(idx))(*idx)))
+    return out
+
+
 class _Optimizer:
     _name = "Optimizer"
 
     def __init__(self, params):
         self.params = list(params)
         self._saved_t = weakref.WeakKeyDictionary()  # store -> this optimizer's step count
+        self._grouped = ([], [])  # the parameters last grouped, and their groups
 
     def _stores(self):
-        return _group_by_store(self.params, self._name)
+        """[(store, members, their sorted indices as the ABI takes them)].  Grouped again
+        whenever `params` no longer holds the same tensors in the same order."""
+        params, groups = self._grouped
+        if len(params) != len(self.params) or not all(map(operator.is_, params, self.params)):
+            groups = _with_indices(_group_by_store(self.params, self._name))
+            self._grouped = (list(self.params), groups)
+        return groups
 
     def _claim(self, store):
         """Make the store's step count this optimizer's before it steps the store.
@@ -71,13 +89,16 @@ class _Optimizer:
         # py/optim.py:89-92 -> Tensor.zero_grad (py/engine.py:141-142): grad = None, and
         # non-Tensor entries are skipped (step() is where they raise).  A store fully owned
         # by this optimizer is cleared with one fill (zeros + no grads).
-        tensors = [p for p in self.params if isinstance(p, Tensor)]
-        for store, members in _group_by_store(tensors, self._name):
+        try:
+            groups = self._stores()
+        except ValueError:  # other entries among the parameters
+            groups = _with_indices(_group_by_store([p for p in self.params
+                                                    if isinstance(p, Tensor)], self._name))
+        for store, members, indices in groups:
             if len(members) == len(store.tensors):
                 store.zero_grad(set_to_none=True)
-            else:
-                for p in members:
-                    p.zero_grad()
+            else:  # each member's `grad = None`
+                store.zero_grad(set_to_none=True, indices=indices, fill=False)
 
     def step(self, tensor_sums=False, update_scale=True):
         """py/optim.py's step().  Extensions: tensor_sums=True takes the gradient norm from
@@ -86,11 +107,10 @@ class _Optimizer:
         of several optimizers stepping one loss-scaled store in an iteration, leaves the loss
         scale to that last step (or to ParamStore.scaler_update()), as torch's
         GradScaler.step(opt) per optimizer followed by one GradScaler.update() does."""
-        for store, members in self._stores():
+        for store, members, indices in self._stores():
             self._claim(store)
             whole = len(members) == len(store.tensors)
-            self._step_store(store, None if whole else sorted({p.index for p in members}),
-                             tensor_sums, update_scale)
+            self._step_store(store, None if whole else indices, tensor_sums, update_scale)
 
     def _step_store(self, store, indices, tensor_sums, update_scale):  # pragma: no cover
         raise NotImplementedError

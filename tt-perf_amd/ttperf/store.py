@@ -12,7 +12,9 @@ from __future__ import annotations
 
 import ctypes as C
 import gc
+import itertools
 import math
+import operator
 import weakref
 
 import numpy as np
@@ -320,6 +322,21 @@ class ParamStore:
     def sync(self):
         L.check(L.lib.ttp_sync(self._h))
 
+    def _shared_stream(self, device):
+        """torch's current stream on `device` where it is the store's own stream too, else None.
+
+        Work on device tensors then needs no synchronisation: it runs behind what torch has
+        queued there, and what torch queues there next runs behind it.  Memory that the
+        tensors' allocator could hand to another stream's work is kept by record_stream.  While
+        torch captures a graph, None: the synchronising form refuses there."""
+        import torch
+        if device.index != self.device or torch.cuda.is_current_stream_capturing():
+            return None
+        s = torch.cuda.current_stream(device)
+        h = C.c_void_p()
+        L.check(L.lib.ttp_get_stream(self._h, C.byref(h)))
+        return s if (h.value or 0) == s.cuda_stream else None
+
     # ---- buffers -----------------------------------------------------------------------------
     def ptr(self, which, index=L.ALL_TENSORS):
         """Device address of a contiguously stored buffer (PARAM, GRAD, MOMENTUM; MASTER in
@@ -373,12 +390,10 @@ class ParamStore:
             if t.element_size() != self._esize(which):
                 raise ValueError("element size does not match the buffer's type")
             kind = L.DEVICE if t.is_cuda else L.HOST
-            if t.is_cuda:
-                import torch
-                torch.cuda.current_stream(t.device).synchronize()
+            shared = self._before_device_source(t) if t.is_cuda else None
             L.check(L.lib.ttp_upload(self._h, which, index, C.c_void_p(t.data_ptr()), n, kind))
             if t.is_cuda:
-                self.sync()  # `t` may be freed and reused by torch as soon as we return
+                self._after_device_sources((t,), shared)
             return
         a = np.asarray(value)
         want = self._host_dtype(which)
@@ -390,6 +405,27 @@ class ParamStore:
         if a.size != n:
             raise ValueError(f"expected {n} elements, got {a.size}")
         L.check(L.lib.ttp_upload(self._h, which, index, a.ctypes.data_as(C.c_void_p), n, L.HOST))
+
+    def _before_device_source(self, t):
+        """Order the store's next work behind torch's on `t`: by the stream they share (which
+        is returned), or by waiting for torch's current stream."""
+        shared = self._shared_stream(t.device)
+        if shared is None:
+            import torch
+            torch.cuda.current_stream(t.device).synchronize()
+        return shared
+
+    def _after_device_sources(self, tensors, shared):
+        """The queued work's sources may be freed by the caller from here on: on a shared stream
+        torch keeps their memory until the work has run, else the work is waited for.  (Writing
+        to them from a third stream takes that stream's wait for the shared one, as behind any
+        torch operation.)"""
+        if shared is None:
+            self.sync()
+            return
+        import torch
+        for _ in map(torch.Tensor.record_stream, tensors, itertools.repeat(shared)):
+            pass
 
     def _check_captured_tensor(self, t, n, which):
         """While capturing, a device transfer becomes a copy node that reads or writes `t`'s
@@ -416,7 +452,7 @@ class ParamStore:
                 raise ValueError(f"out must be a contiguous tensor of {n} elements of "
                                  f"{self._esize(which)} bytes")
             kind = L.DEVICE if out.is_cuda else L.HOST
-            if out.is_cuda:
+            if out.is_cuda and self._shared_stream(out.device) is None:
                 import torch
                 torch.cuda.current_stream(out.device).synchronize()
             L.check(L.lib.ttp_download(self._h, which, index, C.c_void_p(out.data_ptr()), n, kind))
@@ -513,12 +549,11 @@ class ParamStore:
             t = value.detach().contiguous()
             if t.numel() != n:
                 raise ValueError(f"expected {n} elements, got {t.numel()}")
-            if t.is_cuda:
-                torch.cuda.current_stream(t.device).synchronize()
+            shared = self._before_device_source(t) if t.is_cuda else None
             L.check(L.lib.ttp_accumulate_grad(self._h, index, C.c_void_p(t.data_ptr()), n,
                                               dtype | flag, L.DEVICE if t.is_cuda else L.HOST))
             if t.is_cuda:
-                self.sync()  # `t` may be freed and reused by torch as soon as we return
+                self._after_device_sources((t,), shared)
             return
         a = np.asarray(value)
         if a.dtype == np.uint16:
@@ -542,33 +577,51 @@ class ParamStore:
         indices = [int(i) for i in indices]
         if len(values) != len(indices):
             raise ValueError("one value per index")
-        dtypes = {v.dtype for v in values}
-        if not dtypes <= {torch.float32, torch.bfloat16} or len(dtypes) > 1:
-            raise ValueError("incoming gradients must be all float32 or all bfloat16")
+        dtypes = self._bucket_dtypes(indices, values)
         dtype = L.DTYPE_BF16 if dtypes == {torch.bfloat16} else L.DTYPE_F32
-        for i, v in zip(indices, values):
-            # an index out of range is the library's to refuse (TTP_ERR_RANGE), as for a list
-            # that names a tensor twice
-            if 0 <= i < len(self.tensors) and not (
-                    _is_torch(v) and v.is_cuda and v.is_contiguous()
-                    and v.numel() == self.tensors[i].numel):
-                raise ValueError(f"tensor {i}: a contiguous device tensor of "
-                                 f"{self.tensors[i].numel} elements is needed")
+        shared = None
         if not self._in_capture and values:
-            torch.cuda.current_stream(values[0].device).synchronize()
+            shared = self._before_device_source(values[0])
         n = len(indices)
         idx = (C.c_uint32 * max(n, 1))(*indices)
-        ptrs = (C.c_void_p * max(n, 1))(*[v.data_ptr() for v in values])
+        ptrs = (C.c_void_p * max(n, 1))(*map(torch.Tensor.data_ptr, values))
         L.check(L.lib.ttp_accumulate_grad_multi(self._h, idx, ptrs, n,
                                                 dtype | (L.ACCUM_SUMSQ if sums else 0)))
         if not self._in_capture:
-            self.sync()  # the values may be freed and reused by torch as soon as we return
+            self._after_device_sources(values, shared)
+
+    def _bucket_dtypes(self, indices, values):
+        """The values' dtypes, checked with their tensors' element counts (ValueError)."""
+        import torch
+        dtypes = set(map(operator.attrgetter("dtype"), values))
+        if not dtypes <= {torch.float32, torch.bfloat16} or len(dtypes) > 1:
+            raise ValueError("incoming gradients must be all float32 or all bfloat16")
+        t = self.tensors
+        # all in order, each question asked of the whole bucket at once; else one by one, for
+        # the refusal that names the tensor
+        if indices and min(indices) >= 0 and max(indices) < len(t) and \
+                set(map(type, values)) <= {torch.Tensor, torch.nn.Parameter} and \
+                all(map(operator.attrgetter("is_cuda"), values)) and \
+                all(map(torch.Tensor.is_contiguous, values)) and \
+                list(map(torch.Tensor.numel, values)) == [t[i].numel for i in indices]:
+            return dtypes
+        for i, v in zip(indices, values):
+            # an index out of range is the library's to refuse (TTP_ERR_RANGE), as for a list
+            # that names a tensor twice
+            if 0 <= i < len(t) and not (
+                    _is_torch(v) and v.is_cuda and v.is_contiguous()
+                    and v.numel() == t[i].numel):
+                raise ValueError(f"tensor {i}: a contiguous device tensor of "
+                                 f"{t[i].numel} elements is needed")
+        return dtypes
 
     # ---- steps -----------------------------------------------------------------------------------
     @staticmethod
     def _index_array(indices):
         if indices is None:
             return None, 0
+        if isinstance(indices, C.Array):  # a list made once (an optimizer's)
+            return indices, len(indices)
         idx = (C.c_uint32 * max(len(indices), 1))(*[int(i) for i in indices])
         return idx, len(indices)
 
