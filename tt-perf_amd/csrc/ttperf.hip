@@ -220,6 +220,9 @@ struct ttp_ctx {
 
     ttp_scaler_config scaler{0, 2000, 65536.0, 2.0, 0.5};
     uint64_t host_t = 0;     // step count while it lives on the host (see dev_t)
+    // other optimizers' step counts (ttp_swap_step), on the host or the device as the count is
+    uint64_t host_slots[TTP_STEP_SLOTS] = {};
+    uint64_t* slots = nullptr;
     bool device_t = false;   // set once the context has been captured: t stays on the device
     bool capturing = false;  // between ttp_capture_begin and ttp_capture_end
     uint32_t n_graphs = 0;   // live graphs; the buffers and tables they reference stay put
@@ -255,6 +258,16 @@ size_t grad_esize(const ttp_ctx* c) { return bf16_grads(c) ? 2 : 4; }
 // device decides whether a step is skipped) and once the context has been captured (a
 // replayed graph cannot update host state); otherwise on the host.
 bool t_on_device(const ttp_ctx* c) { return c->scaler.enabled || c->device_t; }
+
+// the saved step counts follow the step count between host and device (the stream is idle)
+int move_slots(ttp_ctx* c, bool was_on_device, bool on_device) {
+    if (was_on_device == on_device) return TTP_OK;
+    HIP_TRY(on_device ? hipMemcpy(c->slots, c->host_slots, sizeof(c->host_slots),
+                                  hipMemcpyHostToDevice)
+                      : hipMemcpy(c->host_slots, c->slots, sizeof(c->host_slots),
+                                  hipMemcpyDeviceToHost));
+    return TTP_OK;
+}
 
 int no_capture(const ttp_ctx* c, const char* what) {
     if (!c->capturing) return TTP_OK;
@@ -1149,7 +1162,7 @@ void release(ttp_ctx* c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : {(void*)c->grad, (void*)c->records, (void*)c->momentum, (void*)c->mom_init,
-                    (void*)c->st, (void*)c->partials, (void*)c->tickets, c->staging, (void*)c->tsum,
+                    (void*)c->st, (void*)c->slots, (void*)c->partials, (void*)c->tickets, c->staging, (void*)c->tsum,
                     (void*)c->tile_sums, (void*)c->acc_tiles, (void*)c->tile_base,
                     (void*)c->tsum_pending})
         if (p) (void)hipFree(p);
@@ -1294,6 +1307,7 @@ int ttp_create(int device, const ttp_tensor_desc* descs, uint32_t n, int mode, t
     if ((rc = alloc_zero(c, (void**)&c->mom_init, std::max<uint64_t>(n, 1) * 4))) return bail(rc);
     c->host_mom_init.assign(n, 0);
     if ((rc = alloc_zero(c, (void**)&c->st, sizeof(DevState)))) return bail(rc);
+    if ((rc = alloc_zero(c, (void**)&c->slots, sizeof(c->host_slots)))) return bail(rc);
     c->partials_cap = 2 * c->norm_grid_cap;  // the norm pass's two launches (NormSplit)
     if ((rc = alloc_zero(c, (void**)&c->partials, (uint64_t)c->partials_cap * 8))) return bail(rc);
     if ((rc = alloc_zero(c, (void**)&c->tickets, ttp::kTicketWords * 4))) return bail(rc);
@@ -2266,6 +2280,27 @@ int ttp_set_step(ttp_ctx* c, uint64_t step) {
     return TTP_OK;
 }
 
+int ttp_swap_step(ttp_ctx* c, int save, int load) {
+    int rc = check_ctx(c);
+    if (rc) return rc;
+    if (save < -1 || save >= TTP_STEP_SLOTS || load < -1 || load >= TTP_STEP_SLOTS)
+        return fail(TTP_ERR_RANGE, "a step-count slot is -1 or 0 .. " +
+                                       std::to_string(TTP_STEP_SLOTS - 1));
+    if ((rc = no_capture(c, "ttp_swap_step"))) return rc;
+    if (!t_on_device(c)) {
+        const uint64_t next = load >= 0 ? c->host_slots[load] : 0;
+        if (save >= 0) c->host_slots[save] = c->host_t;
+        c->host_t = next;
+        return TTP_OK;
+    }
+    if ((rc = set_dev(c))) return rc;
+    clear_hip_error();
+    hipLaunchKernelGGL(ttp::swap_step_kernel, dim3(1), dim3(64), 0, c->stream, c->st, c->slots,
+                       (int32_t)save, (int32_t)load);
+    HIP_TRY(hipGetLastError());
+    return TTP_OK;
+}
+
 int ttp_scaler_configure(ttp_ctx* c, const ttp_scaler_config* cfg) {
     int rc = check_ctx(c);
     if (rc) return rc;
@@ -2286,6 +2321,7 @@ int ttp_scaler_configure(ttp_ctx* c, const ttp_scaler_config* cfg) {
     DevState s;
     HIP_TRY(hipMemcpy(&s, c->st, sizeof(s), hipMemcpyDeviceToHost));
     const bool was = t_on_device(c), will = cfg->enabled || c->device_t;
+    if ((rc = move_slots(c, was, will))) return rc;
     if (was && !will) c->host_t = s.t;  // device count -> host
     if (!was && will) s.t = c->host_t;  // host count -> device
     if (cfg->enabled) {
@@ -2607,6 +2643,7 @@ int ttp_load_state(ttp_ctx* c, const char* path) {
                            c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     for (size_t i = 0; i < c->tensors.size(); ++i) c->host_mom_init[i] = (uint8_t)mom[i];
+    if ((rc = move_slots(c, t_on_device(c), h.scaler_enabled || c->device_t))) return rc;
     c->scaler.enabled = h.scaler_enabled;
     c->scaler.growth_interval = h.growth_interval;
     c->scaler.init_scale = h.init_scale;
@@ -2634,6 +2671,7 @@ int ttp_capture_begin(ttp_ctx* c) {
     if ((rc = set_dev(c))) return rc;
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (!t_on_device(c)) {  // from now on the step count lives on the device
+        if ((rc = move_slots(c, false, true))) return rc;
         HIP_TRY(hipMemcpy(&c->st->t, &c->host_t, sizeof(c->host_t), hipMemcpyHostToDevice));
     }
     c->device_t = true;

@@ -23,6 +23,7 @@ DTYPE_F32, DTYPE_BF16 = 0, 1
 ACCUM_SUMSQ = 0x100
 ACCUM_MULTI_MAX = 64  # tensors per ttp_accumulate_grad_multi call
 ZERO_NO_FILL = 0x100  # OR'd into zero_grad's set_to_none: flags only
+STEP_SLOTS = 64  # step counts ttp_swap_step keeps
 STEP_TENSOR_SUMS = 1
 STEP_DEFER_SCALE = 2
 KERNEL_NORM, KERNEL_UPDATE = 0, 1
@@ -98,6 +99,7 @@ SIGNATURES = {
     "ttp_grad_sumsq_tensors": (C.c_int, [_P, C.POINTER(C.c_uint32), C.c_uint32]),
     "ttp_get_step": (C.c_int, [_P, C.POINTER(C.c_uint64)]),
     "ttp_set_step": (C.c_int, [_P, C.c_uint64]),
+    "ttp_swap_step": (C.c_int, [_P, C.c_int, C.c_int]),
     "ttp_scaler_configure": (C.c_int, [_P, C.POINTER(ScalerConfig)]),
     "ttp_scaler_get": (C.c_int, [_P, C.POINTER(C.c_float), C.POINTER(C.c_int32)]),
     "ttp_scaler_set": (C.c_int, [_P, C.c_float, C.c_int32]),

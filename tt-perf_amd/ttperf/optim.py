@@ -13,9 +13,9 @@ AdamW — Adam with decoupled weight decay (p *= 1 - lr*wd before the update), a
 
 Each optimizer counts its own steps, as py/optim.py:46,50 keeps `_step` per Adam, although
 the count the kernels read lives in the store: when a different live optimizer stepped a
-store last, its count is saved and this optimizer's restored (one synchronising read and
-one write, on a change of owner only), so two optimizers over two parameter groups of one
-store see the bias corrections of their own step counts.
+store last, its count is saved in the store and this optimizer's restored (ttp_swap_step, on a
+change of owner only), so two optimizers over two parameter groups of one store see the bias
+corrections of their own step counts.
 
 Every step is one libttperf_hip call per store: one multi-tensor launch (plus the norm pass
 when clipping or loss scaling), instead of ~15 elementwise programs per tensor.
@@ -53,7 +53,8 @@ class _Optimizer:
 
     def __init__(self, params):
         self.params = list(params)
-        self._saved_t = weakref.WeakKeyDictionary()  # store -> this optimizer's step count
+        # store -> where this optimizer's step count is while another's is in the store
+        self._saved_t = weakref.WeakKeyDictionary()
         self._grouped = ([], [])  # the parameters last grouped, and their groups
 
     def _stores(self):
@@ -80,9 +81,13 @@ class _Optimizer:
                 raise RuntimeError(
                     "a second optimizer steps this store inside a graph capture; the step "
                     "count hand-over reads the device and cannot be captured")
-            if prev is not None:
-                prev._saved_t[store] = store.step_count
-            store.step_count = self._saved_t.pop(store, 0)
+            hand_over = getattr(store, "_hand_over_step", None)
+            if hand_over is not None:
+                hand_over(prev, self)
+            else:  # a store that keeps no saved counts: as numbers
+                if prev is not None:
+                    prev._saved_t[store] = (-1, store.step_count)
+                store.step_count = self._saved_t.pop(store, (-1, 0))[1]
         store._t_owner = weakref.ref(self)
 
     def zero_grad(self):

@@ -270,6 +270,7 @@ class ParamStore:
         self._graphs = weakref.WeakSet()
         self._in_capture = False
         self._t_owner = None  # weakref to the optimizer whose step count the store holds
+        self._t_slots = {}  # step-count slot -> weakref to the optimizer whose count it holds
         self._stream_obj = None  # the adopted stream (set_stream), kept alive while in use
 
     # ---- lifetime --------------------------------------------------------------------------
@@ -692,6 +693,31 @@ class ParamStore:
     @step_count.setter
     def step_count(self, t):
         L.check(L.lib.ttp_set_step(self._h, int(t)))
+
+    def _hand_over_step(self, prev, opt):
+        """Save optimizer `prev`'s step count (None: no live optimizer's) and make the store's
+        count `opt`'s: its saved one, or 0.  Each saved count is a slot of the store (of an
+        optimizer that is gone, free again), or a number when the slots are all taken."""
+        save, count = -1, None
+        if prev is not None:
+            for k in range(L.STEP_SLOTS):
+                held = self._t_slots.get(k)
+                if held is None or held() is None:
+                    save = k
+                    break
+            else:
+                count = self.step_count
+        mine = opt._saved_t.pop(self, None)  # (slot, count)
+        load = mine[0] if mine is not None else -1
+        L.check(L.lib.ttp_swap_step(self._h, save, load))
+        if load >= 0:
+            del self._t_slots[load]
+        elif mine is not None:
+            self.step_count = mine[1]
+        if prev is not None:
+            if save >= 0:
+                self._t_slots[save] = weakref.ref(prev)
+            prev._saved_t[self] = (save, count)
 
     def configure_scaler(self, enabled=True, init_scale=2.0 ** 16, growth_factor=2.0,
                          backoff_factor=0.5, growth_interval=2000):
