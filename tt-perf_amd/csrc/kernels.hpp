@@ -174,9 +174,42 @@ __device__ __forceinline__ void st_bf16x4_partial(uint16_t* p, f32x4 v, int n) {
 // ------------------------------------------------------------------------------------
 // block reduction of a double (fixed shape: deterministic)
 // ------------------------------------------------------------------------------------
+// x of the lane that a DPP control names (both 32-bit halves)
+template <int kCtrl>
+__device__ __forceinline__ double dpp(double x) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kCtrl, 0xF, 0xF, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), kCtrl, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, (uint64_t)lo | ((uint64_t)hi << 32));
+}
+
+// The wave's sum in every lane, as the butterfly x += x[lane ^ off] for off = 32, 16, 8, 4, 2, 1
+// gives it (bit for bit), without LDS permutes: a swap of the wave's halves, then of its 16-lane
+// rows; within a row a rotation by 8, then by 4 (the values repeat every 8 lanes by then, so lane
+// + 4 holds what lane ^ 4 does), then quad permutes.  Each LDS permute waited ~100 cycles, twelve
+// of them in a chain at the end of every block: nanoGPT-char's AdamW step took 53.6 us with them
+// and takes 53.2, the last of 8 GPT-2 124M shards 74.3 and 74.0.
 __device__ __forceinline__ double wave_sum(double x) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    {
+        const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)u, false, false);
+        const auto hi =
+            __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+        x = __builtin_bit_cast(double, (uint64_t)lo[0] | ((uint64_t)hi[0] << 32)) +
+            __builtin_bit_cast(double, (uint64_t)lo[1] | ((uint64_t)hi[1] << 32));
+    }
+    {
+        const uint64_t w = __builtin_bit_cast(uint64_t, x);
+        const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)w, (uint32_t)w, false, false);
+        const auto hi =
+            __builtin_amdgcn_permlane16_swap((uint32_t)(w >> 32), (uint32_t)(w >> 32), false, false);
+        x = __builtin_bit_cast(double, (uint64_t)lo[0] | ((uint64_t)hi[0] << 32)) +
+            __builtin_bit_cast(double, (uint64_t)lo[1] | ((uint64_t)hi[1] << 32));
+    }
+    x += dpp<0x128>(x);  // row_ror:8
+    x += dpp<0x124>(x);  // row_ror:4
+    x += dpp<0x4E>(x);   // quad_perm:[2,3,0,1]
+    x += dpp<0xB1>(x);   // quad_perm:[1,0,3,2]
     return x;
 }
 
@@ -1165,7 +1198,7 @@ __global__ __launch_bounds__(kLanes) void sgd_bf16_lane_kernel(const uint16_t* _
 // The sum is the norm pass's bit for bit: each tile's four waves, the tile from its waves, then
 // the tiles in the order of finalize_block.  A step this small
 // is bound by launches and by the chain of round trips in each: at the MLP's 9,610 parameters
-// (fp32 AdamW with clipping, four tiles) it took 9.3 us in two launches and takes 6.1.
+// (fp32 AdamW with clipping, four tiles) it took 9.3 us in two launches and takes 5.7.
 constexpr int kSmallBlock = 1024;
 constexpr uint32_t kSmallTiles = 64;  // at most: one lane of a wave per tile
 
@@ -1179,9 +1212,16 @@ struct SmallArgs {
     uint32_t* tickets;
 };
 
+// Every tile descriptor in one load, a lane each (there are at most 64): a wave reads the ones it
+// needs from there.  A kernel's first load: it waits for nothing but the arguments.
+__device__ __forceinline__ u32x4 small_descs(const SmallArgs& s) {
+    const uint32_t lane = threadIdx.x & 63u;
+    return *reinterpret_cast<const u32x4*>(s.tiles + min(lane, max(s.ntiles, 1u) - 1));
+}
+
 template <typename GradT>
 __device__ __forceinline__ double small_sumsq(const GradT* __restrict__ g, const SmallArgs& s,
-                                              float inv, double* lds) {
+                                              const u32x4& desc, float inv, double* lds) {
     typedef GradVec<GradT> GV;
     typedef typename GV::raw R;
     constexpr int E = GV::kElems;
@@ -1189,38 +1229,51 @@ __device__ __forceinline__ double small_sumsq(const GradT* __restrict__ g, const
     constexpr int kRound = 2;                                // tiles in flight per wave
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t lane = threadIdx.x & 63u;
-    // every descriptor in one load, a lane each; a wave then reads the ones it needs from there
-    const u32x4 desc = *reinterpret_cast<const u32x4*>(s.tiles + min(lane, s.ntiles - 1));
-    for (uint32_t j0 = 0; wave / kWaves + j0 * kTilesAtOnce < s.ntiles; j0 += kRound) {
-        uint32_t tile[kRound], part[kRound], count[kRound];
+    // Goes to the wave's next tile, from the j-th on, that has elements in the wave's part
+    // (uniform; the sums of parts without are 0).  The part moves on with each tile, so that the
+    // first parts, all that short tensors have, are spread over the four waves.
+    uint32_t j = 0;
+    auto next = [&](uint32_t& tile, uint32_t& part, uint32_t& count, uint64_t& begin) {
+        for (;; ++j) {
+            tile = wave / kWaves + j * kTilesAtOnce;
+            part = (wave + j) % kWaves;
+            count = 0;
+            if (tile >= s.ntiles) return false;
+            count = (uint32_t)__builtin_amdgcn_readlane(desc.z, tile);
+            if (part * 64 * E < count) break;
+            if (lane == 0) lds[tile * kWaves + part] = 0.0;
+        }
+        begin = (uint32_t)__builtin_amdgcn_readlane(desc.x, tile) |
+                ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(desc.y, tile) << 32);
+        ++j;
+        return true;
+    };
+    uint32_t tile[kRound], part[kRound], count[kRound];
+    uint64_t begin[kRound];
+    while (next(tile[0], part[0], count[0], begin[0])) {
         R w[kRound][kNormLoads];
+        begin[1] = begin[0];  // no second tile: its loads read this one's start, and count as 0
+        next(tile[1], part[1], count[1], begin[1]);
 #pragma unroll
         for (int u = 0; u < kRound; ++u) {
-            // the wave's part moves on with each tile, so that the first parts, all that short
-            // tensors have, are spread over the four waves
-            tile[u] = wave / kWaves + (j0 + u) * kTilesAtOnce;
-            part[u] = (wave + j0 + u) % kWaves;
-            const uint32_t t = min(tile[u], s.ntiles - 1);
-            const uint64_t begin = (uint32_t)__builtin_amdgcn_readlane(desc.x, t) |
-                                   ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(desc.y, t) << 32);
-            count[u] = tile[u] < s.ntiles ? __builtin_amdgcn_readlane(desc.z, t) : 0u;
 #pragma unroll
             for (int l = 0; l < kNormLoads; ++l) {
-                // (uniform) a wave with nothing below the count reads nothing; a lane's vector
-                // past the count reads the tile's first one, and counts as 0
-                if ((uint32_t)(l * kBlock + part[u] * 64) * E >= count[u]) break;
+                // a lane's vector past the count reads the tile's first one, and counts as 0
                 const uint32_t off = (uint32_t)(l * kBlock + part[u] * 64 + lane) * E;
-                w[u][l] = *reinterpret_cast<const R*>(g + begin + (off < count[u] ? off : 0u));
+                w[u][l] =
+                    *reinterpret_cast<const R*>(g + begin[u] + (off < count[u] ? off : 0u));
             }
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < kRound; ++u) {
-            if (tile[u] >= s.ntiles) break;
+            if (!count[u]) break;
             double acc[2] = {0.0, 0.0};  // as norm_partials_kernel
 #pragma unroll
             for (int l = 0; l < kNormLoads; ++l) {
-                // what is left out here would add zeros, which change no sum
+                // What is left out here would add zeros, which change no sum.  (All of it for
+                // every part, with no branch, took 11.7-13.8 us where this takes 9.5: 60
+                // tensors of 300 elements, whose one wave part each is all there is.)
                 if ((uint32_t)(l * kBlock + part[u] * 64) * E >= count[u]) break;
                 const uint32_t off = (uint32_t)(l * kBlock + part[u] * 64 + lane) * E;
 #pragma unroll
@@ -1229,8 +1282,7 @@ __device__ __forceinline__ double small_sumsq(const GradT* __restrict__ g, const
                     acc[j & 1] = __builtin_fma(x, x, acc[j & 1]);
                 }
             }
-            double sum = 0.0;
-            if (part[u] * 64 * E < count[u]) sum = wave_sum(acc[0] + acc[1]);  // (uniform)
+            const double sum = wave_sum(acc[0] + acc[1]);
             if (lane == 0) lds[tile[u] * kWaves + part[u]] = sum;
         }
     }
@@ -1247,11 +1299,11 @@ struct SmallStep {
 };
 template <typename GradT>
 __device__ __forceinline__ SmallStep small_step(const GradT* __restrict__ g, const SmallArgs& s,
-                                                double* lds) {
+                                                const u32x4& desc, double* lds) {
     SmallStep r;
     r.s0 = *s.fin.st;
     r.bias = load_bias(s.fin, r.s0.t);
-    r.sumsq = s.ntiles ? small_sumsq(g, s, unscale_factor(s.fin, r.s0.scale), lds) : 0.0;
+    r.sumsq = s.ntiles ? small_sumsq(g, s, desc, unscale_factor(s.fin, r.s0.scale), lds) : 0.0;
     r.d = decide(s.fin, r.s0.scale, r.sumsq);
     return r;
 }
@@ -1273,6 +1325,7 @@ __global__ __launch_bounds__(kSmallBlock) void adam_small_kernel(const GradT* __
                                                                  AdamArgs a, SmallArgs s) {
     __shared__ double lds[kSmallTiles * kWaves];
     __shared__ uint32_t last;
+    const u32x4 desc = small_descs(s);
     const Chunk ch = load_chunk(a.chunks, blockIdx.x);
     const bool live = threadIdx.x < ch.count;
     const uint64_t i = ch.begin + threadIdx.x;
@@ -1286,7 +1339,7 @@ __global__ __launch_bounds__(kSmallBlock) void adam_small_kernel(const GradT* __
         m = *mp;
         v = mp[kRec];
     }
-    const SmallStep r = small_step(grad, s, lds);
+    const SmallStep r = small_step(grad, s, desc, lds);
     if (live && !r.d.skip) {
         const bool dev_bias = a.flags & kDevBias;
         const Coefs k{r.d.inv, r.d.coef, dev_bias ? r.bias.next1 : a.bias1,
@@ -1309,6 +1362,7 @@ __global__ __launch_bounds__(kSmallBlock) void sgd_small_kernel(const GradT* __r
                                                                 SgdArgs a, SmallArgs s) {
     __shared__ double lds[kSmallTiles * kWaves];
     __shared__ uint32_t last;
+    const u32x4 desc = small_descs(s);
     const Chunk ch = load_chunk(a.chunks, blockIdx.x);
     const bool live = threadIdx.x < ch.count;
     const bool mom_on = a.flags & kMomOn;
@@ -1321,7 +1375,7 @@ __global__ __launch_bounds__(kSmallBlock) void sgd_small_kernel(const GradT* __r
         p = *pp;
         if (mom_on && !first) b = momentum[i];
     }
-    const SmallStep r = small_step(grad, s, lds);
+    const SmallStep r = small_step(grad, s, desc, lds);
     if (live && !r.d.skip) {
         sgd_elem(p, g, b, a, r.d.inv, r.d.coef, a.flags & kUseInv, a.flags & kUseClip,
                  (ch.meta & kChunkDecay) && (a.flags & kWdOn), mom_on, first,
@@ -1337,6 +1391,7 @@ __global__ __launch_bounds__(kSmallBlock) void sgd_bf16_small_kernel(
     const uint16_t* __restrict__ grad, uint16_t* __restrict__ param, SgdArgs a, SmallArgs s) {
     __shared__ double lds[kSmallTiles * kWaves];
     __shared__ uint32_t last;
+    const u32x4 desc = small_descs(s);
     const Chunk ch = load_chunk(a.chunks, blockIdx.x);
     const bool live = threadIdx.x < ch.count;
     const uint64_t i = ch.begin + threadIdx.x;
@@ -1345,7 +1400,7 @@ __global__ __launch_bounds__(kSmallBlock) void sgd_bf16_small_kernel(
         ld_grad_lane<1>(grad, i, &g);
         ld_grad_lane<1>(param, i, &p);
     }
-    const SmallStep r = small_step(grad, s, lds);
+    const SmallStep r = small_step(grad, s, desc, lds);
     if (live && !r.d.skip)
         param[i] = (uint16_t)bf16_rne(sgd_bf16_elem(p, g, a.lr, r.d.inv, r.d.coef,
                                                     a.flags & kUseInv, a.flags & kUseClip));
