@@ -836,10 +836,12 @@ ttp::SmallArgs small_args(const ttp_ctx* c, const WorkTables* w, bool run_norm,
 // pass's, or that of the pending sums' combination; a launch of its own remains where neither
 // runs.  `probe` only computes the norm.
 // `partials` (null: the context's own) holds one partial per norm-pass block; a caller-given
-// array (the no-allocation step's) also turns the per-launch timing events off.
+// array (the no-allocation step's) also turns the per-launch timing events off.  `stage_marks`:
+// the momentum marks of w's tensors are set there too (see ttp::kMomNew).
 int launch_prologue(ttp_ctx* c, const WorkTables* w, bool run_norm, double max_norm, bool probe,
                     bool want_bias, bool count_t, bool from_sums = false,
-                    bool defer_scale = false, double* partials = nullptr) {
+                    bool defer_scale = false, double* partials = nullptr,
+                    bool stage_marks = false) {
     const NormSplit ns = norm_split(c, w->n_tiles);
     const int32_t scaler_on = c->scaler.enabled ? 1 : 0;
     TimedLaunch tl(c, TTP_KERNEL_NORM, partials == nullptr);
@@ -848,6 +850,11 @@ int launch_prologue(ttp_ctx* c, const WorkTables* w, bool run_norm, double max_n
                                         defer_scale);
     a.partials = partials;
     a.npartials = run_norm ? ns.partials() : 0;
+    if (stage_marks) {
+        a.mom_init = c->mom_init;
+        a.mom_ids = w->tensor_ids;
+        a.n_mom = w->n_tensors;
+    }
     if (run_norm && from_sums) {  // the step's tensors' sums, in tensor order
         a.partials = c->tsum;
         a.idx = w->tensor_ids;
@@ -1990,6 +1997,9 @@ static int adam_step_impl(ttp_ctx* c, const ttp_adam_hparams* hp, const uint32_t
     return TTP_OK;
 }
 
+// most tensors whose momentum marks the decisions' block sets: 16 rounds of its 256 lanes
+constexpr uint32_t kMaxStagedMarks = 4096;
+
 static int sgd_step_impl(ttp_ctx* c, const ttp_sgd_hparams* hp, const uint32_t* subset,
                          uint32_t nsub, ttp_step_report* report) {
     int rc = check_ctx(c);
@@ -2025,20 +2035,23 @@ static int sgd_step_impl(ttp_ctx* c, const ttp_sgd_hparams* hp, const uint32_t* 
     // the momentum buffer once nothing above can refuse the step (a refused call changes
     // nothing, not even what a checkpoint would hold)
     if (mom && (rc = ensure_momentum(c))) return rc;
-    const bool small = one_launch_step(c, w, need_norm || devt, from_sums);
-    if ((need_norm || devt) && !small &&
-        (rc = launch_prologue(c, w, need_norm, hp->max_grad_norm, false, false, devt, from_sums,
-                              defer)))
-        return rc;
-    if (!devt) c->host_t += 1;
     // With momentum, the stepped tensors hold a momentum buffer after the step (torch: state
     // created on first use).  They are marked where the host does not know them marked: with
     // loss scaling the device decides, since the step may be skipped, and once captured the
-    // marking is part of every replay.
+    // marking is part of every replay.  The launch that takes the decisions marks them, as long
+    // as its one block does so in a few rounds; else a launch after the update does (4-5 us at
+    // GPT-2 124M's 121,600 chunks).
     bool mark = mom && (scaler || devt);
     if (mom)
         for (uint32_t i : active)
             if (!c->host_mom_init[i]) mark = true;
+    const bool small = one_launch_step(c, w, need_norm || devt, from_sums);
+    const bool staged = mark && !small && (need_norm || devt) && w->n_tensors <= kMaxStagedMarks;
+    if ((need_norm || devt) && !small &&
+        (rc = launch_prologue(c, w, need_norm, hp->max_grad_norm, false, false, devt, from_sums,
+                              defer, nullptr, staged)))
+        return rc;
+    if (!devt) c->host_t += 1;
 
     ttp::SgdArgs a{};
     a.chunks = chunks;
@@ -2049,7 +2062,7 @@ static int sgd_step_impl(ttp_ctx* c, const ttp_sgd_hparams* hp, const uint32_t* 
     a.wd = (float)hp->weight_decay;
     a.mom_init = c->mom_init;
     a.flags = (hp->weight_decay != 0.0 ? ttp::kWdOn : 0u) | (mom ? ttp::kMomOn : 0u) |
-              (hp->nesterov ? ttp::kNesterov : 0u);
+              (hp->nesterov ? ttp::kNesterov : 0u) | (staged ? ttp::kMomStaged : 0u);
     if (scaler) a.flags |= ttp::kUseInv | ttp::kCheckSkip;
     if (clip) a.flags |= ttp::kUseClip;
     a.st = (need_norm || devt) ? c->st : nullptr;
@@ -2124,7 +2137,7 @@ static int sgd_step_impl(ttp_ctx* c, const ttp_sgd_hparams* hp, const uint32_t* 
 #undef TTP_SGD_LANES
         HIP_TRY(hipGetLastError());
         tl.done();
-        if (mark && !small) {
+        if (mark && !small && !staged) {
             const uint32_t g =
                 std::max<uint32_t>(1, std::min<uint32_t>((n + ttp::kBlock - 1) / ttp::kBlock, 1024));
             clear_hip_error();
@@ -2501,7 +2514,7 @@ int ttp_save_state(ttp_ctx* c, const char* path) {
     };
     bool ok = put(&h, sizeof(h));
     for (size_t i = 0; ok && i < c->tensors.size(); ++i) {
-        StateTensor t{c->tensors[i].numel, c->tensors[i].flags, mom[i]};
+        StateTensor t{c->tensors[i].numel, c->tensors[i].flags, mom[i] ? 1u : 0u};
         ok = put(&t, sizeof(t));
     }
     // each buffer as one contiguous fp32 array, whatever its device layout: gathered into
