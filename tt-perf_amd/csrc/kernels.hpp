@@ -530,7 +530,7 @@ __global__ __launch_bounds__(kBlock) void norm_partials_kernel(const GradT* __re
     for (; c < t1; c += gridDim.x) {
         const R* q = reinterpret_cast<const R*>(g + ch.begin) + threadIdx.x;
         const uint32_t count = ch.count;
-        const uint32_t next = c + gridDim.x;  // (below 2^24 + 2^17 tiles and blocks: no wrap)
+        const uint32_t next = c + gridDim.x;  // (at most 2^28 tiles, 2^17 blocks: no wrap)
         ch = load_chunk(tiles, next < t1 ? next : c);
         if (count == kTile) {
             R w[kNormLoads];
