@@ -6,8 +6,8 @@
  * exp_avg_sq, momentum); the optimizer-private fp32 state is interleaved in records of
  * 64-element slots (see ttp_buffer_layout).  A step over all tensors is one multi-tensor update
  * launch (split in several only beyond 2^32 work-items), plus, when clipping or loss scaling
- * is on, a grad-norm/inf-check pass (one launch, two above 256 MiB of gradients) and a
- * one-block finalize.
+ * is on, a grad-norm/inf-check pass (one launch, two above 256 MiB of gradients); over a small
+ * set both are one launch.
  *
  * Reference interfaces each group of entry points replaces (csirak/tt-perf):
  *   ttp_create / ttp_destroy / ttp_tensor_*  — per-parameter storage owned by

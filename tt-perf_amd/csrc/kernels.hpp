@@ -40,7 +40,7 @@
 
 namespace ttp {
 
-constexpr int kBlock = 256;     // 4 wave64s: norm pass, finalize and helper kernels
+constexpr int kBlock = 256;     // 4 wave64s: norm pass, its decisions and helper kernels
 constexpr int kUpdBlock = 256;  // 4 wave64s: the four-element update
 constexpr int kVec = 4;         // elements per lane per vector
 constexpr uint32_t kChunk = kUpdBlock * kVec;  // 1024 elements: one vector per lane
@@ -86,7 +86,8 @@ __device__ __forceinline__ Chunk load_chunk(const Chunk* t, uint64_t k) {
     return Chunk{(uint64_t)w.x | ((uint64_t)w.y << 32), w.z, w.w};
 }
 
-// Device-resident step state.  Written only by norm_finalize_kernel (and by the host between
+// Device-resident step state.  Written only by the block that decides (write_state), by
+// scaler_update_kernel and by swap_step_kernel (and by the host between
 // steps); read by the update pass that follows it on the same stream.
 struct DevState {
     float scale;             // loss scale (persistent)
@@ -603,7 +604,7 @@ __global__ void swap_step_kernel(DevState* st, uint64_t* slots, int32_t save, in
 // sums[tensor_ids[t]].
 // the sum of tile_sums[b .. e-1] in a fixed order (valid in thread 0): lane l adds tiles
 // b + l, b + l + kBlock, b + l + 2 kBlock, ... in that order, a round of kSumRound of them
-// loaded before their adds (as norm_finalize_kernel), then the fixed block reduction.  One
+// loaded before their adds (as finalize_block), then the fixed block reduction.  One
 // order for every caller, so a tensor's sum does not depend on which call computed its tiles.
 // The round size sets only how many loads are in flight, not the order (tiles past the end
 // add +0.0 to a sum of squares, which leaves it as it is).  A round's loads are unconditional

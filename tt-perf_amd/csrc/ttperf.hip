@@ -14,8 +14,8 @@
 //   * work table: chunks of <= kChunk (1024) elements of one tensor.  The table of all
 //     tensors is built once; a second table is built only while some tensor has no grad
 //     (py/optim.py:56-57 skip);
-//   * step: [norm pass (partials + finalize) when clipping or loss scaling] + one fused
-//     update pass, all on the context's stream, no host synchronisation (the skip decision
+//   * step: [norm pass, whose last block decides, when clipping or loss scaling] + one fused
+//     update pass (one launch for both over small tensor sets), all on the context's stream, no host synchronisation (the skip decision
 //     and, with loss scaling, the step count live on the device).
 #include <hip/hip_runtime.h>
 
