@@ -857,30 +857,36 @@ __device__ __forceinline__ void st_lane(float* p, const float* v, int n) {
         }
     }
 }
-template <int kE>
+// the bf16 copies of the first n (1..kE) of kE values, non-temporal or (kNT false) ordinary
+template <bool kNT, typename T>
+__device__ __forceinline__ void st_word(T* p, T w) {
+    if constexpr (kNT) __builtin_nontemporal_store(w, p);
+    else *p = w;
+}
+template <int kE, bool kNT = true>
 __device__ __forceinline__ void st_bf16_lane(uint16_t* p, const float* v, int n) {
     if constexpr (kE == 1) {
-        __builtin_nontemporal_store((uint16_t)bf16_rne(v[0]), p);
+        st_word<kNT>(p, (uint16_t)bf16_rne(v[0]));
     } else if constexpr (kE == 2) {
         if (n == 2)
-            __builtin_nontemporal_store(bf16_pack(v[0], v[1]), reinterpret_cast<uint32_t*>(p));
+            st_word<kNT>(reinterpret_cast<uint32_t*>(p), bf16_pack(v[0], v[1]));
         else
-            __builtin_nontemporal_store((uint16_t)bf16_rne(v[0]), p);
+            st_word<kNT>(p, (uint16_t)bf16_rne(v[0]));
     } else {
         if (n == 4) {
-            __builtin_nontemporal_store(u32x2{bf16_pack(v[0], v[1]), bf16_pack(v[2], v[3])},
-                                        reinterpret_cast<u32x2*>(p));
+            st_word<kNT>(reinterpret_cast<u32x2*>(p),
+                         u32x2{bf16_pack(v[0], v[1]), bf16_pack(v[2], v[3])});
         } else {
 #pragma unroll
             for (int j = 0; j < 3; ++j)
-                if (j < n) __builtin_nontemporal_store((uint16_t)bf16_rne(v[j]), p + j);
+                if (j < n) st_word<kNT>(p + j, (uint16_t)bf16_rne(v[j]));
         }
     }
 }
 
 // One piece of the lane-form Adam update: this lane's kE elements at flat index i (the first
 // n of them stored: a tensor's last piece may end inside the lane).
-template <typename GradT, bool kMixed, int kE>
+template <typename GradT, bool kMixed, int kE, bool kCopyNT>
 __device__ __forceinline__ void adam_piece(const GradT* __restrict__ grad,
                                            float* __restrict__ records, float* __restrict__ master,
                                            uint16_t* __restrict__ param16, const AdamArgs& a,
@@ -901,7 +907,7 @@ __device__ __forceinline__ void adam_piece(const GradT* __restrict__ grad,
     st_lane<kE>(pp, p, n);
     st_lane<kE>(mp, m, n);
     st_lane<kE>(vp, v, n);
-    if (kMixed) st_bf16_lane<kE>(param16 + i, p, n);
+    if (kMixed) st_bf16_lane<kE, kCopyNT>(param16 + i, p, n);
 }
 
 // The lane-form Adam update: one block per part of kIt consecutive pieces of kLanes x kE
@@ -912,8 +918,9 @@ __device__ __forceinline__ void adam_piece(const GradT* __restrict__ grad,
 // per block, and halves the grid a skipped step dispatches.  records is the record array's
 // base ([master|m|v] in MIXED, [m|v] in FP32), master the contiguous FP32 weights (unused in
 // MIXED).  a.st must be valid: its fields are read unconditionally and used as a.flags say.
-// The arithmetic is adam_elem's, so every shape gives the same results bit for bit.
-template <typename GradT, bool kMixed, int kE, int kLanes, int kIt>
+// The arithmetic is adam_elem's, so every shape gives the same results bit for bit.  kCopyNT: the
+// bf16 copy is stored non-temporally (see kCachedCopyElems in ttperf.hip).
+template <typename GradT, bool kMixed, int kE, int kLanes, int kIt, bool kCopyNT = true>
 __global__ __launch_bounds__(kLanes) void adam_lane_kernel(const GradT* __restrict__ grad,
                                                            float* __restrict__ records,
                                                            float* __restrict__ master,
@@ -935,7 +942,7 @@ __global__ __launch_bounds__(kLanes) void adam_lane_kernel(const GradT* __restri
     const bool use_inv = a.flags & kUseInv, use_clip = a.flags & kUseClip;
     const bool decay = (ch.meta & kChunkDecay) && (a.flags & kWdOn);
     if constexpr (kIt == 1) {
-        adam_piece<GradT, kMixed, kE>(grad, records, master, param16, a, k, use_inv, use_clip,
+        adam_piece<GradT, kMixed, kE, kCopyNT>(grad, records, master, param16, a, k, use_inv, use_clip,
                                       decay, ch.begin + off,
                                       (int)min(ch.count - off, (uint32_t)kE));
     } else {
@@ -943,7 +950,7 @@ __global__ __launch_bounds__(kLanes) void adam_lane_kernel(const GradT* __restri
         for (int q = 0; q < kIt; ++q) {
             const uint32_t o = off + q * kPiece;
             if (o >= ch.count) break;
-            adam_piece<GradT, kMixed, kE>(grad, records, master, param16, a, k, use_inv,
+            adam_piece<GradT, kMixed, kE, kCopyNT>(grad, records, master, param16, a, k, use_inv,
                                           use_clip, decay, ch.begin + o,
                                           (int)min(ch.count - o, (uint32_t)kE));
         }

@@ -690,6 +690,13 @@ constexpr uint32_t kMaxGridBlocks = 1u << 22;
 // back and after a gradient copy (3.476 against 3.472 ms, 4.095 against 4.089 ms), and
 // dispatches twice the workgroups on a skipped step.
 constexpr int kLaneAdamMixedCached = 1, kLanesAdamMixedCached = 128, kItAdamMixedCached = 2;
+// Up to this many elements the cached MIXED Adam shape stores the bf16 copy with ordinary stores,
+// which the Infinity Cache takes beside the gradients (100 MB of both at the line); beyond, they
+// push out the gradients that the norm pass left there, and non-temporal stores are faster.
+// AdamW steps in us, ordinary / non-temporal: 4M elements 25.7 / 26.1, nanoGPT-char's 10.8M
+// 52.7 / 53.4, 15.6M 73.8 / 74.7, 23M 102.6 / 103.3, 31M 143.5 / 142.8, 62M 281 / 275,
+// 124M 565 / 543.
+constexpr uint64_t kCachedCopyElems = 24ull << 20;
 constexpr int kLaneAdamMixed = 1, kLanesAdamMixed = 256, kItAdamMixed = 2;
 constexpr int kLaneAdamFp32 = 1, kLanesAdamFp32 = 128, kItAdamFp32 = 2;
 constexpr int kLaneSgdMixed = 1, kLanesSgdMixed = 256, kItSgdMixed = 2;
@@ -1956,7 +1963,18 @@ static int adam_step_impl(ttp_ctx* c, const ttp_adam_hparams* hp, const uint32_t
                 hipLaunchKernelGGL((ttp::adam_small_kernel<float, false>), dim3(n),
                                    dim3(ttp::kSmallBlock), 0, c->stream, g32, c->records,
                                    c->master, (uint16_t*)nullptr, a, s);
-        } else if (grads_cached(c, w) && c->mode == TTP_MODE_MIXED)
+        } else if (c->mode == TTP_MODE_MIXED && w->elems <= kCachedCopyElems)
+            launch_lanes(c,
+                         (uint64_t)n * ttp::lane_parts<kLaneAdamMixedCached, kLanesAdamMixedCached,
+                                                       kItAdamMixedCached>(),
+                         kLanesAdamMixedCached, [&](dim3 g, uint64_t p0) {
+                hipLaunchKernelGGL(
+                    (ttp::adam_lane_kernel<uint16_t, true, kLaneAdamMixedCached,
+                                           kLanesAdamMixedCached, kItAdamMixedCached, false>), g,
+                    dim3(kLanesAdamMixedCached), 0, c->stream, g16, c->records, (float*)nullptr,
+                    p16, al, p0);
+            });
+        else if (grads_cached(c, w) && c->mode == TTP_MODE_MIXED)
             launch_lanes(c,
                          (uint64_t)n * ttp::lane_parts<kLaneAdamMixedCached, kLanesAdamMixedCached,
                                                        kItAdamMixedCached>(),
