@@ -1,0 +1,99 @@
+"""Which device sources upload, accumulate_grad and accumulate_grads return before reading: those
+whose memory torch's caching allocator keeps for the shared stream (record_stream).  Memory that
+torch only wraps is waited for, as its owner may reuse it.  CPU: the tensors pass for device
+tensors, and the library and the streams are stand-ins that note what was called."""
+import types
+
+import numpy as np
+import pytest
+import torch
+
+import ttperf
+from ttperf import store as S
+
+N = 64
+
+
+class _Device(torch.Tensor):
+    """A host tensor that passes for one of cuda:0 (and for a type of torch's)."""
+
+    __module__ = "torch"
+
+    is_cuda = property(lambda self: True)
+    device = property(lambda self: torch.device("cuda", 0))
+
+
+def _tensor(memory):
+    if memory == "torch":
+        return torch.zeros(N)
+    if memory == "a torch slice":
+        return torch.zeros(4 * N)[N:2 * N]
+    if memory == "an array":  # as from an array interface: wrapped, not allocated
+        return torch.from_numpy(np.zeros(N, np.float32))
+    return torch.utils.dlpack.from_dlpack(torch.utils.dlpack.to_dlpack(torch.zeros(N)))
+
+
+def _call(store, entry, sources):
+    if entry == "upload":
+        store.upload(ttperf.BUF_GRAD, 0, sources[0])
+    elif entry == "accumulate":
+        store.accumulate_grad(0, sources[0])
+    else:
+        store.accumulate_grads(list(range(len(sources))), sources)
+
+
+@pytest.fixture
+def bench(monkeypatch):
+    log = []
+
+    def entry(name):
+        return lambda *a: log.append(name) or 0
+
+    names = ("ttp_upload", "ttp_accumulate_grad", "ttp_accumulate_grad_multi", "ttp_sync",
+             "ttp_destroy")
+    monkeypatch.setattr(S.L, "lib", types.SimpleNamespace(**{n: entry(n) for n in names}))
+    stream = types.SimpleNamespace(synchronize=lambda: log.append("torch waits"))
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: stream)
+    monkeypatch.setattr(torch.Tensor, "record_stream",
+                        lambda self, s: log.append(("kept", self.untyped_storage().data_ptr())))
+    st = S.ParamStore.__new__(S.ParamStore)
+    st._h, st.mode, st.device, st._in_capture = None, S.L.MODE_FP32, 0, False
+    st.tensors = [S.Tensor(st, i, (N,)) for i in range(3)]
+    st.total = 3 * N
+    monkeypatch.setattr(S.ParamStore, "_shared_stream", lambda self, device: stream)
+    return st, log
+
+
+@pytest.mark.parametrize("entry", ["upload", "accumulate", "bucket"])
+@pytest.mark.parametrize("memory", ["torch", "a torch slice", "an array", "dlpack"])
+def test_only_torchs_own_memory_is_left_unread(bench, entry, memory):
+    st, log = bench
+    src = _tensor(memory).as_subclass(_Device)
+    _call(st, entry, [src])
+    if memory.startswith(("torch", "a torch")):
+        assert len(log) == 2 and log[0].startswith("ttp_")  # queued, nothing waited for
+        assert log[1] == ("kept", src.untyped_storage().data_ptr())
+    else:
+        assert log[-1] == "ttp_sync" and log[-2] in ("ttp_upload", "ttp_accumulate_grad",
+                                                     "ttp_accumulate_grad_multi")
+
+
+def test_a_bucket_with_one_wrapped_source_is_waited_for(bench):
+    st, log = bench
+    _call(st, "bucket", [_tensor(m).as_subclass(_Device) for m in ("torch", "dlpack", "torch")])
+    assert log[-2:] == ["ttp_accumulate_grad_multi", "ttp_sync"]
+
+
+def test_each_storage_is_kept_once(bench):
+    st, log = bench
+    base, alone = torch.zeros(2 * N), torch.zeros(N)
+    _call(st, "bucket", [t.as_subclass(_Device) for t in (base[:N], alone, base[N:])])
+    assert log[0] == "ttp_accumulate_grad_multi" and \
+        sorted(log[1:]) == sorted(("kept", t.data_ptr()) for t in (base, alone))
+
+
+def test_a_pluggable_allocator_is_not_relied_on(bench, monkeypatch):
+    st, log = bench
+    monkeypatch.setattr(torch.cuda, "get_allocator_backend", lambda: "pluggable")
+    _call(st, "accumulate", [_tensor("torch").as_subclass(_Device)])
+    assert log[-1] == "ttp_sync"

@@ -96,3 +96,51 @@ def test_an_edited_parameter_list_is_grouped_again():
         opt.step()
     opt.zero_grad()
     store.close()
+
+
+@pytest.mark.parametrize("entry", ["upload", "accumulate", "bucket"])
+def test_sources_that_torch_only_wraps(entry):
+    """Read before the call returns, so that their owner may write to them or take them back:
+    another store's view, which that store overwrites on its own stream, and an array interface
+    over memory that goes back to another stream's pool."""
+    import ttperf
+    from ttperf.store import _torch_storages
+    torch = torch_mod()
+    a = torch.randn(4096, 4096, device="cuda")
+    store = ttperf.ParamStore([(N,)], mode="fp32")
+    store.set_stream(torch.cuda.current_stream())
+    second = ttperf.ParamStore([(N,)], mode="fp32")  # on its own stream
+    view = second.torch_view(ttperf.BUF_GRAD, 0)
+    other = torch.cuda.Stream()
+    assert _torch_storages([view]) is None and _torch_storages([a[:2], view]) is None
+    assert [t.data_ptr() for t in _torch_storages([a[1:], a[:1]])] == [a[:1].data_ptr()]
+
+    def busy():
+        for _ in range(20):
+            a @ a
+
+    for k in range(3):
+        second.upload(ttperf.BUF_GRAD, 0, torch.full((N,), k + 1.0, device="cuda"))
+        busy()
+        _hand_over(store, entry, view)
+        second.zero_grad()
+        assert (store.download(ttperf.BUF_GRAD, 0) == k + 1.0).all()
+        with torch.cuda.stream(other):
+            owner = torch.full((N,), k + 10.0, device="cuda")
+
+            class Wrapped:
+                __cuda_array_interface__ = dict(owner.__cuda_array_interface__)
+
+            src = torch.as_tensor(Wrapped(), device="cuda")
+            ptr = owner.data_ptr()
+            assert src.data_ptr() == ptr
+        torch.cuda.current_stream().wait_stream(other)
+        busy()
+        _hand_over(store, entry, src)
+        del src, owner
+        with torch.cuda.stream(other):
+            again = torch.full((N,), -2.0, device="cuda")
+        assert (store.download(ttperf.BUF_GRAD, 0) == k + 10.0).all(), ptr == again.data_ptr()
+    torch.cuda.synchronize()
+    store.close()
+    second.close()

@@ -12,7 +12,6 @@ from __future__ import annotations
 
 import ctypes as C
 import gc
-import itertools
 import math
 import operator
 import weakref
@@ -24,6 +23,20 @@ from . import _lib as L
 
 def _is_torch(x):
     return type(x).__module__.startswith("torch")
+
+
+def _torch_storages(tensors):
+    """One tensor per distinct storage of `tensors` where Tensor.record_stream keeps each of those
+    storages for a stream's work, else None.  It keeps what torch's own caching allocator handed
+    out.  Memory that torch only wraps (DLPack, __cuda_array_interface__, another process's, a
+    store's torch_view) it leaves alone without a word: its owner may take it back or write to it
+    at any time.  Wrapped storages cannot be resized, the allocator's can; a pluggable allocator
+    keeps memory only if it was made to."""
+    import torch
+    if torch.cuda.get_allocator_backend() == "pluggable":
+        return None
+    storages = dict(zip(map(torch.Tensor.untyped_storage, tensors), tensors))
+    return list(storages.values()) if all(s.resizable() for s in storages) else None
 
 
 def _bf16_bits_to_f32(h):
@@ -327,9 +340,8 @@ class ParamStore:
         """torch's current stream on `device` where it is the store's own stream too, else None.
 
         Work on device tensors then needs no synchronisation: it runs behind what torch has
-        queued there, and what torch queues there next runs behind it.  Memory that the
-        tensors' allocator could hand to another stream's work is kept by record_stream.  While
-        torch captures a graph, None: the synchronising form refuses there."""
+        queued there, and what torch queues there next runs behind it.  While torch captures a
+        graph, None: the synchronising form refuses there."""
         import torch
         if device.index != self.device or torch.cuda.is_current_stream_capturing():
             return None
@@ -391,10 +403,10 @@ class ParamStore:
             if t.element_size() != self._esize(which):
                 raise ValueError("element size does not match the buffer's type")
             kind = L.DEVICE if t.is_cuda else L.HOST
-            shared = self._before_device_source(t) if t.is_cuda else None
+            kept = self._before_device_sources((t,)) if t.is_cuda else None
             L.check(L.lib.ttp_upload(self._h, which, index, C.c_void_p(t.data_ptr()), n, kind))
             if t.is_cuda:
-                self._after_device_sources((t,), shared)
+                self._after_device_sources(kept)
             return
         a = np.asarray(value)
         want = self._host_dtype(which)
@@ -407,26 +419,30 @@ class ParamStore:
             raise ValueError(f"expected {n} elements, got {a.size}")
         L.check(L.lib.ttp_upload(self._h, which, index, a.ctypes.data_as(C.c_void_p), n, L.HOST))
 
-    def _before_device_source(self, t):
-        """Order the store's next work behind torch's on `t`: by the stream they share (which
-        is returned), or by waiting for torch's current stream."""
-        shared = self._shared_stream(t.device)
-        if shared is None:
+    def _before_device_sources(self, tensors):
+        """Order the store's next work behind torch's on `tensors` (all of one device): on the
+        stream both share, where torch keeps the sources until that work has run, else by waiting
+        for torch's current stream.  Returns what _after_device_sources takes."""
+        device = tensors[0].device
+        shared = self._shared_stream(device)
+        keep = _torch_storages(tensors) if shared is not None else None
+        if keep is None:
             import torch
-            torch.cuda.current_stream(t.device).synchronize()
-        return shared
+            torch.cuda.current_stream(device).synchronize()
+            return None
+        return shared, keep
 
-    def _after_device_sources(self, tensors, shared):
-        """The queued work's sources may be freed by the caller from here on: on a shared stream
-        torch keeps their memory until the work has run, else the work is waited for.  (Writing
-        to them from a third stream takes that stream's wait for the shared one, as behind any
-        torch operation.)"""
-        if shared is None:
+    def _after_device_sources(self, kept):
+        """From here on the caller may free the sources of the work just queued: torch keeps their
+        memory until it has run, or (`kept` None) it is waited for.  (Writing to a kept source
+        from a third stream takes that stream's wait for the shared one, as behind any torch
+        operation.)"""
+        if kept is None:
             self.sync()
             return
-        import torch
-        for _ in map(torch.Tensor.record_stream, tensors, itertools.repeat(shared)):
-            pass
+        shared, keep = kept
+        for t in keep:
+            t.record_stream(shared)
 
     def _check_captured_tensor(self, t, n, which):
         """While capturing, a device transfer becomes a copy node that reads or writes `t`'s
@@ -550,11 +566,11 @@ class ParamStore:
             t = value.detach().contiguous()
             if t.numel() != n:
                 raise ValueError(f"expected {n} elements, got {t.numel()}")
-            shared = self._before_device_source(t) if t.is_cuda else None
+            kept = self._before_device_sources((t,)) if t.is_cuda else None
             L.check(L.lib.ttp_accumulate_grad(self._h, index, C.c_void_p(t.data_ptr()), n,
                                               dtype | flag, L.DEVICE if t.is_cuda else L.HOST))
             if t.is_cuda:
-                self._after_device_sources((t,), shared)
+                self._after_device_sources(kept)
             return
         a = np.asarray(value)
         if a.dtype == np.uint16:
@@ -580,16 +596,16 @@ class ParamStore:
             raise ValueError("one value per index")
         dtypes = self._bucket_dtypes(indices, values)
         dtype = L.DTYPE_BF16 if dtypes == {torch.bfloat16} else L.DTYPE_F32
-        shared = None
+        kept = None
         if not self._in_capture and values:
-            shared = self._before_device_source(values[0])
+            kept = self._before_device_sources(values)
         n = len(indices)
         idx = (C.c_uint32 * max(n, 1))(*indices)
         ptrs = (C.c_void_p * max(n, 1))(*map(torch.Tensor.data_ptr, values))
         L.check(L.lib.ttp_accumulate_grad_multi(self._h, idx, ptrs, n,
                                                 dtype | (L.ACCUM_SUMSQ if sums else 0)))
         if not self._in_capture:
-            self._after_device_sources(values, shared)
+            self._after_device_sources(kept)
 
     def _bucket_dtypes(self, indices, values):
         """The values' dtypes, checked with their tensors' element counts (ValueError)."""
