@@ -49,10 +49,14 @@ def bench(monkeypatch):
     def entry(name):
         return lambda *a: log.append(name) or 0
 
-    names = ("ttp_upload", "ttp_accumulate_grad", "ttp_accumulate_grad_multi", "ttp_sync",
+    names = ("ttp_download", "ttp_upload", "ttp_accumulate_grad", "ttp_accumulate_grad_multi", "ttp_sync",
              "ttp_destroy")
-    monkeypatch.setattr(S.L, "lib", types.SimpleNamespace(**{n: entry(n) for n in names}))
-    stream = types.SimpleNamespace(synchronize=lambda: log.append("torch waits"))
+    lib = types.SimpleNamespace(**{n: entry(n) for n in names})
+    lib.ttp_get_stream = lambda h, out: asked.append("ttp_get_stream") or 0
+    asked = []
+    monkeypatch.setattr(S.L, "lib", lib)
+    stream = types.SimpleNamespace(synchronize=lambda: log.append("torch waits"),
+                                   device_index=0, cuda_stream=0)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: stream)
     monkeypatch.setattr(torch.Tensor, "record_stream",
                         lambda self, s: log.append(("kept", self.untyped_storage().data_ptr())))
@@ -60,7 +64,9 @@ def bench(monkeypatch):
     st._h, st.mode, st.device, st._in_capture = None, S.L.MODE_FP32, 0, False
     st.tensors = [S.Tensor(st, i, (N,)) for i in range(3)]
     st.total = 3 * N
-    monkeypatch.setattr(S.ParamStore, "_shared_stream", lambda self, device: stream)
+    st.asked = asked
+    st._stream_handle = 0  # adopted: the store's stream and torch's are both the default one
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     return st, log
 
 
@@ -97,3 +103,17 @@ def test_a_pluggable_allocator_is_not_relied_on(bench, monkeypatch):
     monkeypatch.setattr(torch.cuda, "get_allocator_backend", lambda: "pluggable")
     _call(st, "accumulate", [_tensor("torch").as_subclass(_Device)])
     assert log[-1] == "ttp_sync"
+
+
+@pytest.mark.parametrize("entry", ["upload", "accumulate", "bucket", "download"])
+def test_a_store_on_its_own_stream_asks_nothing(bench, entry):
+    """Its calls are torch's wait, the work and the store's wait, with no question to the library
+    or about captures between them."""
+    st, log = bench
+    st._stream_handle = None
+    src = _tensor("torch").as_subclass(_Device)
+    if entry == "download":
+        st.download(ttperf.BUF_GRAD, 0, out=src)
+    else:
+        _call(st, entry, [src])
+    assert log[0] == "torch waits" and log[2:] == ["ttp_sync"] and not st.asked

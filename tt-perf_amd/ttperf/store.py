@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes as C
 import gc
+import itertools
 import math
 import operator
 import weakref
@@ -36,7 +37,9 @@ def _torch_storages(tensors):
     if torch.cuda.get_allocator_backend() == "pluggable":
         return None
     storages = dict(zip(map(torch.Tensor.untyped_storage, tensors), tensors))
-    return list(storages.values()) if all(s.resizable() for s in storages) else None
+    if not all(map(torch.UntypedStorage.resizable, storages)):
+        return None
+    return list(storages.values())
 
 
 def _bf16_bits_to_f32(h):
@@ -285,6 +288,7 @@ class ParamStore:
         self._t_owner = None  # weakref to the optimizer whose step count the store holds
         self._t_slots = {}  # step-count slot -> weakref to the optimizer whose count it holds
         self._stream_obj = None  # the adopted stream (set_stream), kept alive while in use
+        self._stream_handle = None  # and its handle (None: the context's own stream)
 
     # ---- lifetime --------------------------------------------------------------------------
     def close(self):
@@ -325,10 +329,11 @@ class ParamStore:
         default stream); None returns to the context's own stream."""
         if stream is None:
             L.check(L.lib.ttp_reset_stream(self._h))
-            self._stream_obj = None
+            self._stream_obj = self._stream_handle = None
             return
-        handle = stream.cuda_stream if hasattr(stream, "cuda_stream") else stream
-        L.check(L.lib.ttp_set_stream(self._h, C.c_void_p(int(handle))))
+        handle = int(stream.cuda_stream if hasattr(stream, "cuda_stream") else stream)
+        L.check(L.lib.ttp_set_stream(self._h, C.c_void_p(handle)))
+        self._stream_handle = handle
         # the store queues work on this stream until it moves or closes: keep the object
         # (a torch.cuda.Stream, say) alive as long
         self._stream_obj = stream
@@ -336,19 +341,21 @@ class ParamStore:
     def sync(self):
         L.check(L.lib.ttp_sync(self._h))
 
-    def _shared_stream(self, device):
-        """torch's current stream on `device` where it is the store's own stream too, else None.
+    def _torch_stream(self, device):
+        """torch's current stream on `device`, and whether it is the store's too.
 
         Work on device tensors then needs no synchronisation: it runs behind what torch has
-        queued there, and what torch queues there next runs behind it.  While torch captures a
-        graph, None: the synchronising form refuses there."""
+        queued there, and what torch queues there next runs behind it.  Not while torch captures
+        a graph: the synchronising form refuses there.  The library is asked only about the
+        stream set_stream() adopted (asked on every stream, each call took 3 us longer)."""
         import torch
-        if device.index != self.device or torch.cuda.is_current_stream_capturing():
-            return None
-        s = torch.cuda.current_stream(device)
+        stream = torch.cuda.current_stream(device)
+        if stream.cuda_stream != self._stream_handle or stream.device_index != self.device:
+            return stream, False
         h = C.c_void_p()
         L.check(L.lib.ttp_get_stream(self._h, C.byref(h)))
-        return s if (h.value or 0) == s.cuda_stream else None
+        return stream, ((h.value or 0) == self._stream_handle and
+                        not torch.cuda.is_current_stream_capturing())
 
     # ---- buffers -----------------------------------------------------------------------------
     def ptr(self, which, index=L.ALL_TENSORS):
@@ -423,14 +430,12 @@ class ParamStore:
         """Order the store's next work behind torch's on `tensors` (all of one device): on the
         stream both share, where torch keeps the sources until that work has run, else by waiting
         for torch's current stream.  Returns what _after_device_sources takes."""
-        device = tensors[0].device
-        shared = self._shared_stream(device)
-        keep = _torch_storages(tensors) if shared is not None else None
+        stream, shared = self._torch_stream(tensors[0].device)
+        keep = _torch_storages(tensors) if shared else None
         if keep is None:
-            import torch
-            torch.cuda.current_stream(device).synchronize()
+            stream.synchronize()
             return None
-        return shared, keep
+        return stream, keep
 
     def _after_device_sources(self, kept):
         """From here on the caller may free the sources of the work just queued: torch keeps their
@@ -440,9 +445,10 @@ class ParamStore:
         if kept is None:
             self.sync()
             return
-        shared, keep = kept
-        for t in keep:
-            t.record_stream(shared)
+        import torch
+        stream, keep = kept
+        for _ in map(torch.Tensor.record_stream, keep, itertools.repeat(stream)):
+            pass
 
     def _check_captured_tensor(self, t, n, which):
         """While capturing, a device transfer becomes a copy node that reads or writes `t`'s
@@ -469,9 +475,10 @@ class ParamStore:
                 raise ValueError(f"out must be a contiguous tensor of {n} elements of "
                                  f"{self._esize(which)} bytes")
             kind = L.DEVICE if out.is_cuda else L.HOST
-            if out.is_cuda and self._shared_stream(out.device) is None:
-                import torch
-                torch.cuda.current_stream(out.device).synchronize()
+            if out.is_cuda:
+                stream, shared = self._torch_stream(out.device)
+                if not shared:
+                    stream.synchronize()
             L.check(L.lib.ttp_download(self._h, which, index, C.c_void_p(out.data_ptr()), n, kind))
             if kind == L.DEVICE:
                 self.sync()
@@ -614,9 +621,9 @@ class ParamStore:
         if not dtypes <= {torch.float32, torch.bfloat16} or len(dtypes) > 1:
             raise ValueError("incoming gradients must be all float32 or all bfloat16")
         t = self.tensors
-        # all in order, each question asked of the whole bucket at once; else one by one, for
-        # the refusal that names the tensor
-        if indices and min(indices) >= 0 and max(indices) < len(t) and \
+        # all in order, each question asked of the whole bucket at once (which takes longer for a
+        # few tensors); else one by one, for the refusal that names the tensor
+        if len(indices) > 4 and min(indices) >= 0 and max(indices) < len(t) and \
                 set(map(type, values)) <= {torch.Tensor, torch.nn.Parameter} and \
                 all(map(operator.attrgetter("is_cuda"), values)) and \
                 all(map(torch.Tensor.is_contiguous, values)) and \
