@@ -11,6 +11,7 @@ import sys
 import pytest
 
 from conftest import REPO
+from ttperf.store import _StepSlots
 
 HEADER = os.path.join(REPO, "include", "ttperf", "ttperf.h")
 
@@ -181,16 +182,18 @@ def test_non_tensor_params_raise_at_step_and_are_skipped_by_zero_grad():
             opt.step()
 
 
-class _CountingStore:
-    """Stands in for a ParamStore: a step count that every step advances, and a count of the
-    synchronising reads and writes of it."""
+class _CountingStore(_StepSlots):
+    """Stands in for a ParamStore: a step count that every step advances, its slots, and a count
+    of the synchronising reads and writes of it.  Which count goes where is the store's own
+    bookkeeping."""
 
     def __init__(self, n):
         import ttperf
+        super().__init__()
         self.mode = ttperf._lib.MODE_MIXED
         self._t = 0
         self.reads = self.writes = 0
-        self._t_owner = None
+        self.slots = [0] * ttperf._lib.STEP_SLOTS
         self._in_capture = False
         self.tensors = [ttperf.Tensor(self, i, (4,)) for i in range(n)]
         self.log = []
@@ -204,6 +207,12 @@ class _CountingStore:
     def step_count(self, t):
         self.writes += 1
         self._t = t
+
+    def _swap_step(self, save, load):
+        assert -1 <= save < len(self.slots) and -1 <= load < len(self.slots)
+        t, self._t = self._t, self.slots[load] if load >= 0 else 0
+        if save >= 0:
+            self.slots[save] = t
 
     def adam_step(self, lr, betas, eps, weight_decay, decoupled, max_grad_norm, indices=None,
                   tensor_sums=False, update_scale=True):
@@ -248,12 +257,35 @@ def test_each_optimizer_keeps_its_own_step_count():
     assert s.log == [(4.0, 42)]
     b.step()
     assert s.log[-1] == (2.0, 5)
-    # a hand-over reads the device, which a graph capture cannot hold
+    # a hand-over happens once, which a graph capture cannot hold
     s._in_capture = True
     with pytest.raises(RuntimeError, match="capture"):
         d.step()
     b.step()  # no hand-over: fine while capturing
     assert s.log[-1] == (2.0, 6)
+
+
+@pytest.mark.parametrize("live", [2, 64, 65, 66, 130])
+def test_step_counts_beyond_the_slots_and_of_optimizers_that_are_gone(live):
+    """Up to 64 live optimizers (as many as slots) hand their counts over without a read; with
+    more, some keep numbers.  An optimizer that is gone gives its slot back."""
+    import random
+    import ttperf
+    s = _CountingStore(1)
+    r = random.Random(live)
+    opts = [ttperf.Adam(s.tensors, lr=1.0) for _ in range(live)]
+    want = [0] * live
+    for k in range(6 * live):
+        i = k if k < live else r.randrange(live)
+        if k > live and r.random() < 0.1:
+            # (a store whose last optimizer is gone keeps its count for the next one: another's)
+            if s._t_owner() is opts[i]:
+                continue
+            opts[i], want[i] = ttperf.Adam(s.tensors, lr=1.0), 0
+        opts[i].step()
+        want[i] += 1
+        assert s.log[-1] == (1.0, want[i]), k
+    assert (s.reads == 0) == (live <= len(s.slots))
 
 
 def test_cpp_dropin_headers_compile():

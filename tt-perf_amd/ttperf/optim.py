@@ -80,14 +80,8 @@ class _Optimizer:
             if store._in_capture:
                 raise RuntimeError(
                     "a second optimizer steps this store inside a graph capture; the step "
-                    "count hand-over reads the device and cannot be captured")
-            hand_over = getattr(store, "_hand_over_step", None)
-            if hand_over is not None:
-                hand_over(prev, self)
-            else:  # a store that keeps no saved counts: as numbers
-                if prev is not None:
-                    prev._saved_t[store] = (-1, store.step_count)
-                store.step_count = self._saved_t.pop(store, (-1, 0))[1]
+                    "count hand-over happens once and cannot be captured")
+            store._hand_over_step(prev, self)
         store._t_owner = weakref.ref(self)
 
     def zero_grad(self):

@@ -239,7 +239,42 @@ class TraceContext:
     reset = release
 
 
-class ParamStore:
+class _StepSlots:
+    """Which optimizer's step count is where: the one that stepped a store last has its count in
+    the store (_t_owner), others' are in slots of the store (_t_slots: slot -> weakref to the
+    optimizer) or numbers of their own.  A store has `step_count` and `_swap_step(save, load)`."""
+
+    def __init__(self):
+        self._t_owner = None  # weakref to the optimizer whose step count the store holds
+        self._t_slots = {}  # step-count slot -> weakref to the optimizer whose count it holds
+
+    def _hand_over_step(self, prev, opt):
+        """Save optimizer `prev`'s step count (None: no live optimizer's) and make the store's
+        count `opt`'s: its saved one, or 0.  Each saved count is a slot of the store (of an
+        optimizer that is gone, free again), or a number when the slots are all taken."""
+        save, count = -1, None
+        if prev is not None:
+            for k in range(L.STEP_SLOTS):
+                held = self._t_slots.get(k)
+                if held is None or held() is None:
+                    save = k
+                    break
+            else:
+                count = self.step_count
+        mine = opt._saved_t.pop(self, None)  # (slot, count)
+        load = mine[0] if mine is not None else -1
+        self._swap_step(save, load)
+        if load >= 0:
+            del self._t_slots[load]
+        elif mine is not None:
+            self.step_count = mine[1]
+        if prev is not None:
+            if save >= 0:
+                self._t_slots[save] = weakref.ref(prev)
+            prev._saved_t[self] = (save, count)
+
+
+class ParamStore(_StepSlots):
     """One context: tensors laid out 64-element aligned in caller order.
 
     shapes : list of shapes (tuples) or element counts
@@ -285,8 +320,7 @@ class ParamStore:
         self.total = tot.value
         self._graphs = weakref.WeakSet()
         self._in_capture = False
-        self._t_owner = None  # weakref to the optimizer whose step count the store holds
-        self._t_slots = {}  # step-count slot -> weakref to the optimizer whose count it holds
+        _StepSlots.__init__(self)
         self._stream_obj = None  # the adopted stream (set_stream), kept alive while in use
         self._stream_handle = None  # and its handle (None: the context's own stream)
 
@@ -717,30 +751,8 @@ class ParamStore:
     def step_count(self, t):
         L.check(L.lib.ttp_set_step(self._h, int(t)))
 
-    def _hand_over_step(self, prev, opt):
-        """Save optimizer `prev`'s step count (None: no live optimizer's) and make the store's
-        count `opt`'s: its saved one, or 0.  Each saved count is a slot of the store (of an
-        optimizer that is gone, free again), or a number when the slots are all taken."""
-        save, count = -1, None
-        if prev is not None:
-            for k in range(L.STEP_SLOTS):
-                held = self._t_slots.get(k)
-                if held is None or held() is None:
-                    save = k
-                    break
-            else:
-                count = self.step_count
-        mine = opt._saved_t.pop(self, None)  # (slot, count)
-        load = mine[0] if mine is not None else -1
+    def _swap_step(self, save, load):
         L.check(L.lib.ttp_swap_step(self._h, save, load))
-        if load >= 0:
-            del self._t_slots[load]
-        elif mine is not None:
-            self.step_count = mine[1]
-        if prev is not None:
-            if save >= 0:
-                self._t_slots[save] = weakref.ref(prev)
-            prev._saved_t[self] = (save, count)
 
     def configure_scaler(self, enabled=True, init_scale=2.0 ** 16, growth_factor=2.0,
                          backoff_factor=0.5, growth_interval=2000):
