@@ -288,6 +288,38 @@ def test_step_counts_beyond_the_slots_and_of_optimizers_that_are_gone(live):
     assert (s.reads == 0) == (live <= len(s.slots))
 
 
+@pytest.mark.parametrize("where", ["slot", "number"])
+def test_a_refused_hand_over_keeps_every_step_count(where):
+    """The library refuses it (a capture, a lost device): nothing has moved, and the counts are
+    there when it works again."""
+    import ttperf
+    s = _CountingStore(1)
+    if where == "number":
+        s.slots = []
+        ttperf._lib.STEP_SLOTS, slots = 0, ttperf._lib.STEP_SLOTS
+    try:
+        a, b = (ttperf.Adam(s.tensors, lr=1.0) for _ in range(2))
+        for opt in (a, a, b):
+            opt.step()
+
+        def refuse(*args):
+            raise ttperf.TTPError(4, "refused")
+
+        s._swap_step = refuse
+        for opt in (a, a, ttperf.Adam(s.tensors, lr=1.0)):
+            with pytest.raises(ttperf.TTPError):
+                opt.step()
+        assert s._t == 1
+        b.step()  # still the owner
+        del s._swap_step
+        for opt in (a, b, a):
+            opt.step()
+        assert [t for _, t in s.log[-4:]] == [2, 3, 3, 4]
+    finally:
+        if where == "number":
+            ttperf._lib.STEP_SLOTS = slots
+
+
 def test_cpp_dropin_headers_compile():
     """The C++ drop-in tests and bench program (tests/cpp) build against include/ and the
     library."""

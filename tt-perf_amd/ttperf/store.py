@@ -261,17 +261,18 @@ class _StepSlots:
                     break
             else:
                 count = self.step_count
-        mine = opt._saved_t.pop(self, None)  # (slot, count)
-        load = mine[0] if mine is not None else -1
-        self._swap_step(save, load)
-        if load >= 0:
-            del self._t_slots[load]
-        elif mine is not None:
-            self.step_count = mine[1]
+        load, number = opt._saved_t.get(self, (-1, 0))
+        self._swap_step(save, load)  # what it refuses changes nothing here
         if prev is not None:
             if save >= 0:
                 self._t_slots[save] = weakref.ref(prev)
             prev._saved_t[self] = (save, count)
+        self._t_owner = None  # until `opt` steps
+        if load >= 0:
+            del self._t_slots[load]
+        elif number:
+            self.step_count = number
+        opt._saved_t.pop(self, None)
 
 
 class ParamStore(_StepSlots):
