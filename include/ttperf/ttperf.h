@@ -413,7 +413,7 @@ int ttp_set_step(ttp_ctx* ctx, uint64_t step);
 /* Hand the context's step count from one optimizer over its tensors to another, in stream order
  * and without a synchronisation: the count goes to slot `save` (-1: nowhere) and becomes slot
  * `load`'s (-1: 0).  Slots 0 .. TTP_STEP_SLOTS - 1 hold counts, 0 at first, wherever the context
- * counts (host or device).  Not while capturing. */
+ * counts (host or device).  Not while capturing, nor while a caller captures the stream. */
 #define TTP_STEP_SLOTS 64
 int ttp_swap_step(ttp_ctx* ctx, int save, int load);
 /* ttp_scaler_configure also resets the scale to init_scale and the tracker to 0.  Captured

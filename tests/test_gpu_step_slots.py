@@ -55,3 +55,32 @@ def test_slots_out_of_range_are_refused():
         L.check(L.lib.ttp_swap_step(store.handle, 0, 1))
     store.end_capture(discard=True)
     store.close()
+
+
+@pytest.mark.filterwarnings("ignore:The CUDA Graph is empty")
+@pytest.mark.parametrize("scaler", [False, True])
+def test_a_capture_of_the_callers_refuses_the_hand_over(scaler):
+    """A capture that is torch's, not the store's, would replay a hand-over that happened once.
+    Refused, it leaves both counts as they were."""
+    import ttperf
+    torch = torch_mod()
+    store = ttperf.ParamStore([(64,)] * 2, mode="mixed")
+    side = torch.cuda.Stream()
+    store.set_stream(side)
+    if scaler:
+        store.configure_scaler(True, init_scale=8.0)
+    store.upload(ttperf.BUF_GRAD, ttperf.ALL_TENSORS,
+                 torch.ones(store.total, device="cuda", dtype=torch.bfloat16))
+    a, b = (ttperf.AdamW([t], lr=1e-3) for t in store.parameters())
+    for opt in (a, a, b):
+        opt.step()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        with pytest.raises(ttperf.TTPError):
+            a.step()
+    assert store.step_count == 1  # b's
+    a.step()
+    assert store.step_count == 3
+    b.step()
+    assert store.step_count == 2
+    store.close()

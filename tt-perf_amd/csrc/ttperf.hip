@@ -273,6 +273,15 @@ int no_capture(const ttp_ctx* c, const char* what) {
     if (!c->capturing) return TTP_OK;
     return fail(TTP_ERR_STATE, std::string(what) + " is not allowed while capturing a graph");
 }
+// The same for a capture of the context's stream that is not the context's own (its caller's,
+// torch's), of which only the stream knows.
+int no_stream_capture(const ttp_ctx* c, const char* what) {
+    if (!c->stream) return TTP_OK;  // the legacy default stream cannot be captured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(c->stream, &status));
+    if (status == hipStreamCaptureStatusNone) return TTP_OK;
+    return fail(TTP_ERR_STATE, std::string(what) + " is not allowed while its stream is captured");
+}
 size_t param_esize(const ttp_ctx* c) { return bf16_grads(c) ? 2 : 4; }
 
 uint32_t norm_tile(const ttp_ctx* c) {
@@ -2318,6 +2327,8 @@ int ttp_swap_step(ttp_ctx* c, int save, int load) {
         return fail(TTP_ERR_RANGE, "a step-count slot is -1 or 0 .. " +
                                        std::to_string(TTP_STEP_SLOTS - 1));
     if ((rc = no_capture(c, "ttp_swap_step"))) return rc;
+    // every replay would swap the counts again, which the caller's slots would know nothing of
+    if ((rc = no_stream_capture(c, "ttp_swap_step"))) return rc;
     if (!t_on_device(c)) {
         const uint64_t next = load >= 0 ? c->host_slots[load] : 0;
         if (save >= 0) c->host_slots[save] = c->host_t;
