@@ -91,3 +91,42 @@ def test_every_kernel_is_in_the_assembly(isa):
               "norm_finalize_kernel", "accumulate_grad_tiles_kernel",
               "combine_pending_sums_kernel", "tensor_sums_kernel"):
         assert re.search(r"^_ZN3ttp\d+" + k, text, re.M), k
+
+
+def test_what_the_deciding_block_shares_is_not_restrict():
+    """The kernels whose last block decides read and write the step state and the partial sums
+    through FinalizeArgs: another pointer of theirs to the same memory, promised to be the only
+    one, would let the compiler move its accesses past the ticket."""
+    text = open(os.path.join(PKG, "csrc", "kernels.hpp")).read()
+    found = 0
+    for m in re.finditer(r"__global__[^;{]*?\b(\w+_kernel)\(([^;{]*?FinalizeArgs \w+[^;{]*)\)\s*{",
+                         text):
+        found += 1
+        for arg in m.group(2).split(","):
+            if "double*" in arg and "const" not in arg or "DevState*" in arg:
+                assert "__restrict__" not in arg, (m.group(1), arg.strip())
+    assert found >= 3, found
+
+
+def test_a_partial_is_acknowledged_before_its_ticket(isa):
+    """In every kernel that takes tickets: the store of a partial sum (device scope), a wait for
+    all stores, then the ticket."""
+    order, fn = {}, None
+    for line in isa["ttperf.s"]:
+        m = re.match(r"^(_Z\S+):", line)
+        if m:
+            fn = m.group(1)
+        elif fn and re.match(r"^\s*global_store_dwordx2 .*\bsc1\b", line):
+            order.setdefault(fn, []).append("store")
+        elif fn and re.match(r"^\s*s_waitcnt .*vmcnt\(0\).*lgkmcnt\(0\)", line):
+            order.setdefault(fn, []).append("wait")
+        elif fn and re.match(r"^\s*global_atomic_add\b", line):
+            order.setdefault(fn, []).append("ticket")
+    takers = {f: o for f, o in order.items() if "ticket" in o}
+    assert sum("norm_partials_kernel" in f for f in takers) == 2
+    assert sum("combine_pending_sums_kernel" in f for f in takers) == 1
+    assert sum("_small_kernel" in f for f in takers) == 6
+    for f, o in takers.items():
+        before = o[:o.index("ticket")]
+        assert before[-1] == "wait" and "store" not in o[o.index("ticket"):], (f, o)
+        assert ("store" in before) == ("_small_kernel" not in f), (f, o)

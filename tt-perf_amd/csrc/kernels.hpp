@@ -499,13 +499,15 @@ constexpr uint32_t norm_tile_elems() {
 // loads throughout, the update unchanged).  Each block writes one partial, and with kDecide the
 // launch's last block combines all of them (an earlier launch's included) and decides.  Squares
 // of fp32 values are exact in fp64, and any inf/NaN gradient makes the sum non-finite.
+// st and partials are not __restrict__: the deciding block writes the one and reads the other
+// through fin.
 template <typename GradT, bool kNT, bool kDecide>
 __global__ __launch_bounds__(kBlock) void norm_partials_kernel(const GradT* __restrict__ g,
                                                                const Chunk* __restrict__ tiles,
                                                                uint32_t t0, uint32_t t1,
-                                                               const DevState* __restrict__ st,
+                                                               const DevState* st,
                                                                int32_t scaler_on,
-                                                               double* __restrict__ partials,
+                                                               double* partials,
                                                                FinalizeArgs fin,
                                                                uint32_t* __restrict__ tickets) {
     typedef GradVec<GradT> GV;
@@ -660,11 +662,12 @@ __device__ __forceinline__ double tile_from_waves(const double* __restrict__ w, 
 // partials of its tiles, from kWaves x tile_base[tensor]), if it has any pending: each tile
 // from its waves, then the tiles in sum_tiles' order, so the tensor's sum equals what
 // ttp_grad_sumsq_tensors gives for the same gradients.  One launch per step instead of one
-// per accumulate; its last block combines the sums of all stepped tensors and decides.
+// per accumulate; its last block combines the sums of all stepped tensors and decides (it reads
+// them through fin, so sums is not __restrict__).
 __global__ __launch_bounds__(kBlock) void combine_pending_sums_kernel(
     const double* __restrict__ acc_waves, const uint32_t* __restrict__ tile_base,
     const uint32_t* __restrict__ tile_start, const uint32_t* __restrict__ tensor_ids,
-    uint32_t* __restrict__ pending, double* __restrict__ sums, FinalizeArgs fin,
+    uint32_t* __restrict__ pending, double* sums, FinalizeArgs fin,
     uint32_t* __restrict__ tickets) {
     __shared__ double lds[kBlock / 64];
     __shared__ uint32_t last;
