@@ -320,6 +320,17 @@ def test_a_refused_hand_over_keeps_every_step_count(where):
             ttperf._lib.STEP_SLOTS = slots
 
 
+@pytest.mark.parametrize("make", [list, tuple, C.c_uint32 * 2, C.c_int64 * 2, C.c_uint8 * 2,
+                                  C.c_double * 2])
+def test_index_lists_of_any_type_reach_the_library_as_uint32(make):
+    from ttperf import store as S
+    values = (2, 0)
+    given = make(*values) if isinstance(make, type(C.c_uint32 * 2)) else make(values)
+    idx, n = S.ParamStore._index_array(given)
+    C.POINTER(C.c_uint32).from_param(idx)  # as the calls take it
+    assert n == 2 and [idx[0], idx[1]] == [2, 0]
+
+
 def test_cpp_dropin_headers_compile():
     """The C++ drop-in tests and bench program (tests/cpp) build against include/ and the
     library."""

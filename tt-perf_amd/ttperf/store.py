@@ -679,8 +679,8 @@ class ParamStore(_StepSlots):
     def _index_array(indices):
         if indices is None:
             return None, 0
-        if isinstance(indices, C.Array):  # a list made once (an optimizer's)
-            return indices, len(indices)
+        if isinstance(indices, C.Array) and indices._type_ is C.c_uint32:
+            return indices, len(indices)  # a list made once (an optimizer's)
         idx = (C.c_uint32 * max(len(indices), 1))(*[int(i) for i in indices])
         return idx, len(indices)
 
