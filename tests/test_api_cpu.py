@@ -320,6 +320,38 @@ def test_a_refused_hand_over_keeps_every_step_count(where):
             ttperf._lib.STEP_SLOTS = slots
 
 
+@pytest.mark.parametrize("edit", ["cleared", "replaced", "one store of two", "optimizer gone"])
+def test_an_optimizer_keeps_no_store_it_no_longer_steps(edit):
+    """Whatever an optimizer remembers of its parameters, a store is freed once the parameter list
+    holds none of its tensors, before any further call."""
+    import gc
+    import weakref
+    import ttperf
+    s, other = _CountingStore(3), _CountingStore(2)
+    opt = ttperf.Adam(s.tensors + (other.tensors if edit == "one store of two" else []), lr=1.0)
+    opt.step()
+    opt.step()
+    assert [t for _, t in s.log] == [1, 2]
+    if edit == "cleared":
+        opt.params.clear()
+    elif edit == "replaced":
+        opt.params = other.tensors
+    elif edit == "one store of two":
+        opt.params[:] = other.tensors
+    else:
+        store, gone = s, weakref.ref(opt)
+        del opt
+        gc.collect()
+        assert gone() is None and store.log
+        return
+    gone = weakref.ref(s)
+    del s
+    gc.collect()
+    assert gone() is None
+    opt.step()
+    assert len(other.log) == {"cleared": 0, "replaced": 1, "one store of two": 3}[edit]
+
+
 @pytest.mark.parametrize("make", [list, tuple, C.c_uint32 * 2, C.c_int64 * 2, C.c_uint8 * 2,
                                   C.c_double * 2])
 def test_index_lists_of_any_type_reach_the_library_as_uint32(make):

@@ -48,6 +48,16 @@ def _with_indices(groups):
     return out
 
 
+class _Grouping:
+    """The parameters an optimizer last grouped, and their groups.  Held by the one store they
+    are all of, so that it goes when that store does: an optimizer keeps no store alive that its
+    `params` no longer names."""
+    __slots__ = ("params", "groups", "__weakref__")
+
+    def __init__(self, params, groups):
+        self.params, self.groups = params, groups
+
+
 class _Optimizer:
     _name = "Optimizer"
 
@@ -55,15 +65,21 @@ class _Optimizer:
         self.params = list(params)
         # store -> where this optimizer's step count is while another's is in the store
         self._saved_t = weakref.WeakKeyDictionary()
-        self._grouped = ([], [])  # the parameters last grouped, and their groups
+        self._grouped = lambda: None  # weakref to the last _Grouping
 
     def _stores(self):
         """[(store, members, their sorted indices as the ABI takes them)].  Grouped again
-        whenever `params` no longer holds the same tensors in the same order."""
-        params, groups = self._grouped
-        if len(params) != len(self.params) or not all(map(operator.is_, params, self.params)):
-            groups = _with_indices(_group_by_store(self.params, self._name))
-            self._grouped = (list(self.params), groups)
+        whenever `params` no longer holds the same tensors in the same order, and every time over
+        several stores."""
+        kept = self._grouped()
+        if kept is not None and len(kept.params) == len(self.params) and \
+                all(map(operator.is_, kept.params, self.params)):
+            return kept.groups
+        groups = _with_indices(_group_by_store(self.params, self._name))
+        if len(groups) == 1:
+            kept = _Grouping(list(self.params), groups)
+            groups[0][0]._groupings[self] = kept
+            self._grouped = weakref.ref(kept)
         return groups
 
     def _claim(self, store):

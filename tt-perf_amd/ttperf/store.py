@@ -240,11 +240,14 @@ class TraceContext:
 
 
 class _StepSlots:
-    """Which optimizer's step count is where: the one that stepped a store last has its count in
-    the store (_t_owner), others' are in slots of the store (_t_slots: slot -> weakref to the
-    optimizer) or numbers of their own.  A store has `step_count` and `_swap_step(save, load)`."""
+    """What optimizers keep in a store.
+
+    Which one's step count is where: the one that stepped a store last has its count in the store
+    (_t_owner), others' are in slots of the store (_t_slots: slot -> weakref to the optimizer) or
+    numbers of their own.  A store has `step_count` and `_swap_step(save, load)`."""
 
     def __init__(self):
+        self._groupings = weakref.WeakKeyDictionary()  # optimizer -> its parameters, grouped
         self._t_owner = None  # weakref to the optimizer whose step count the store holds
         self._t_slots = {}  # step-count slot -> weakref to the optimizer whose count it holds
 
