@@ -945,17 +945,17 @@ __global__ __launch_bounds__(kLanes) void adam_lane_kernel(const GradT* __restri
     const bool use_inv = a.flags & kUseInv, use_clip = a.flags & kUseClip;
     const bool decay = (ch.meta & kChunkDecay) && (a.flags & kWdOn);
     if constexpr (kIt == 1) {
-        adam_piece<GradT, kMixed, kE, kCopyNT>(grad, records, master, param16, a, k, use_inv, use_clip,
-                                      decay, ch.begin + off,
-                                      (int)min(ch.count - off, (uint32_t)kE));
+        adam_piece<GradT, kMixed, kE, kCopyNT>(grad, records, master, param16, a, k, use_inv,
+                                               use_clip, decay, ch.begin + off,
+                                               (int)min(ch.count - off, (uint32_t)kE));
     } else {
 #pragma unroll 1
         for (int q = 0; q < kIt; ++q) {
             const uint32_t o = off + q * kPiece;
             if (o >= ch.count) break;
             adam_piece<GradT, kMixed, kE, kCopyNT>(grad, records, master, param16, a, k, use_inv,
-                                          use_clip, decay, ch.begin + o,
-                                          (int)min(ch.count - o, (uint32_t)kE));
+                                                   use_clip, decay, ch.begin + o,
+                                                   (int)min(ch.count - o, (uint32_t)kE));
         }
     }
 }

@@ -27,6 +27,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -704,7 +705,10 @@ constexpr int kLaneAdamMixedCached = 1, kLanesAdamMixedCached = 128, kItAdamMixe
 // push out the gradients that the norm pass left there, and non-temporal stores are faster.
 // AdamW steps in us, ordinary / non-temporal: 4M elements 25.7 / 26.1, nanoGPT-char's 10.8M
 // 52.7 / 53.4, 15.6M 73.8 / 74.7, 23M 102.6 / 103.3, 31M 143.5 / 142.8, 62M 281 / 275,
-// 124M 565 / 543.
+// 124M 565 / 543.  Steps without a norm pass take the same line: after a copy of the gradients
+// (copy included) 4M 24.4 / 24.7, 8M 41.5 / 42.5, 15.6M 75.2 / 76.3, 23.5M 110 / 112; back to
+// back within 1% either way from 5M to 14M, 23.5M 97.6 / 99.5; a bucket with its sums and the
+// step from them 4M 33.2 / 33.5, 8M 54.1 / 55.6, 23.5M 124 / 126.
 constexpr uint64_t kCachedCopyElems = 24ull << 20;
 constexpr int kLaneAdamMixed = 1, kLanesAdamMixed = 256, kItAdamMixed = 2;
 constexpr int kLaneAdamFp32 = 1, kLanesAdamFp32 = 128, kItAdamFp32 = 2;
@@ -1972,29 +1976,24 @@ static int adam_step_impl(ttp_ctx* c, const ttp_adam_hparams* hp, const uint32_t
                 hipLaunchKernelGGL((ttp::adam_small_kernel<float, false>), dim3(n),
                                    dim3(ttp::kSmallBlock), 0, c->stream, g32, c->records,
                                    c->master, (uint16_t*)nullptr, a, s);
-        } else if (c->mode == TTP_MODE_MIXED && w->elems <= kCachedCopyElems)
-            launch_lanes(c,
-                         (uint64_t)n * ttp::lane_parts<kLaneAdamMixedCached, kLanesAdamMixedCached,
-                                                       kItAdamMixedCached>(),
-                         kLanesAdamMixedCached, [&](dim3 g, uint64_t p0) {
-                hipLaunchKernelGGL(
-                    (ttp::adam_lane_kernel<uint16_t, true, kLaneAdamMixedCached,
-                                           kLanesAdamMixedCached, kItAdamMixedCached, false>), g,
-                    dim3(kLanesAdamMixedCached), 0, c->stream, g16, c->records, (float*)nullptr,
-                    p16, al, p0);
-            });
-        else if (grads_cached(c, w) && c->mode == TTP_MODE_MIXED)
-            launch_lanes(c,
-                         (uint64_t)n * ttp::lane_parts<kLaneAdamMixedCached, kLanesAdamMixedCached,
-                                                       kItAdamMixedCached>(),
-                         kLanesAdamMixedCached, [&](dim3 g, uint64_t p0) {
-                hipLaunchKernelGGL(
-                    (ttp::adam_lane_kernel<uint16_t, true, kLaneAdamMixedCached,
-                                           kLanesAdamMixedCached, kItAdamMixedCached>), g,
-                    dim3(kLanesAdamMixedCached), 0, c->stream, g16, c->records, (float*)nullptr,
-                    p16, al, p0);
-            });
-        else if (c->mode == TTP_MODE_MIXED)
+        } else if (grads_cached(c, w) && c->mode == TTP_MODE_MIXED) {
+            auto cached = [&](auto copy_nt) {
+                launch_lanes(c,
+                             (uint64_t)n * ttp::lane_parts<kLaneAdamMixedCached,
+                                                           kLanesAdamMixedCached,
+                                                           kItAdamMixedCached>(),
+                             kLanesAdamMixedCached, [&](dim3 g, uint64_t p0) {
+                    hipLaunchKernelGGL(
+                        (ttp::adam_lane_kernel<uint16_t, true, kLaneAdamMixedCached,
+                                               kLanesAdamMixedCached, kItAdamMixedCached,
+                                               decltype(copy_nt)::value>), g,
+                        dim3(kLanesAdamMixedCached), 0, c->stream, g16, c->records,
+                        (float*)nullptr, p16, al, p0);
+                });
+            };
+            if (w->elems <= kCachedCopyElems) cached(std::false_type{});
+            else cached(std::true_type{});
+        } else if (c->mode == TTP_MODE_MIXED)
             launch_lanes(c,
                          (uint64_t)n *
                              ttp::lane_parts<kLaneAdamMixed, kLanesAdamMixed, kItAdamMixed>(),
