@@ -38,6 +38,9 @@ HBM_PEAK_GBPS = 8000.0  # MI355X HBM3E
 # and picks its update form accordingly (kCachedGradBytes in tt-perf_amd/csrc/ttperf.hip):
 # names the kernel in the roofline
 CACHED_GRAD_BYTES = 256 << 20
+# elements up to which MIXED Adam's cached shape stores the bf16 copy with ordinary stores
+# (kCachedCopyElems there)
+CACHED_COPY_ELEMS = 24 << 20
 # algorithmic bytes per parameter of one update-kernel pass (and of the norm pass)
 UPDATE_BYTES = {("adamw", "mixed"): 28, ("adamw", "fp32"): 28, ("sgdm", "fp32"): 20,
                 ("sgdm", "mixed"): 20, ("sgd", "mixed"): 12, ("sgd", "fp32"): 12,
@@ -526,20 +529,25 @@ def step_fn(store, optimizer, hp):
 
 
 def update_kernel_name(optimizer, mode, total_elems, layout="default"):
-    """The update instantiation libttperf_hip launches for a store (its rocprof name): the lane
-    form with its elements per lane, lanes per block and pieces per block (kLaneAdamMixed ...
-    in tt-perf_amd/csrc/ttperf.hip; the SGD forms also with their master's record stride, 64
-    for a contiguous master), except while the gradients fit the Infinity Cache: MIXED Adam
-    then takes the kLaneAdamMixedCached shape, and MIXED SGD momentum in the default layout the
-    four-element kernel; a BF16 store's plain SGD its own kernel (kLaneSgdBf16)."""
+    """The update instantiation that per-kernel timing times for a store (its rocprof name): the
+    lane form with its elements per lane, lanes per block and pieces per block (kLaneAdamMixed
+    ... in tt-perf_amd/csrc/ttperf.hip; the SGD forms also with their master's record stride, 64
+    for a contiguous master, the Adam forms with whether the bf16 copy is stored
+    non-temporally), except while the gradients fit the Infinity Cache: MIXED Adam then takes
+    the kLaneAdamMixedCached shape, and MIXED SGD momentum in the default layout the
+    four-element kernel; a BF16 store's plain SGD its own kernel (kLaneSgdBf16).  (Without
+    per-kernel timing, a clipped or loss-scaled step of at most 32,768 elements in 64 norm tiles
+    has no update launch of its own: adam_small_kernel, sgd_small_kernel and
+    sgd_bf16_small_kernel take the whole step.)"""
     if mode == "bf16":
         return "sgd_bf16_lane_kernel<8, 64, 1>"
     grad_t, mixed_t = ("unsigned short", "true") if mode == "mixed" else ("float", "false")
     if optimizer == "adamw":
         if mode == "mixed" and total_elems * 2 <= CACHED_GRAD_BYTES:
-            return f"adam_lane_kernel<{grad_t}, {mixed_t}, 1, 128, 2>"
+            copy_nt = "false" if total_elems <= CACHED_COPY_ELEMS else "true"
+            return f"adam_lane_kernel<{grad_t}, {mixed_t}, 1, 128, 2, {copy_nt}>"
         e, ln, it = (1, 256, 2) if mode == "mixed" else (1, 128, 2)
-        return f"adam_lane_kernel<{grad_t}, {mixed_t}, {e}, {ln}, {it}>"
+        return f"adam_lane_kernel<{grad_t}, {mixed_t}, {e}, {ln}, {it}, true>"
     contiguous = mode == "fp32" or layout == "sgd"
     stride = "64u" if contiguous else "192u"
     if optimizer == "sgdm" and not contiguous and total_elems * 2 <= CACHED_GRAD_BYTES:

@@ -137,3 +137,24 @@ def compare_state(store, ref, which=("master", "exp_avg", "exp_avg_sq", "param")
             assert worst <= max_ulp, f"{name}: max {worst} ulp (> {max_ulp}), {nbad} values differ"
         del got
     return out
+
+
+def captured_launches(store, call):
+    """How many nodes the store's work in `call` makes in a captured graph, one per launch.  The
+    store must be on a created stream; the capture is discarded."""
+    import ctypes as C
+    from ttperf import _lib as L
+    hip = C.CDLL("libamdhip64.so.7")
+    stream, status, ident = C.c_void_p(), C.c_int(), C.c_ulonglong()
+    graph, nodes = C.c_void_p(), C.c_size_t()
+    L.check(L.lib.ttp_get_stream(store.handle, C.byref(stream)))
+    store.begin_capture()
+    try:
+        call()
+        rc = hip.hipStreamGetCaptureInfo_v2(stream, C.byref(status), C.byref(ident),
+                                            C.byref(graph), None, None)
+        assert rc == 0 and status.value == 1 and graph.value, (rc, status.value)
+        assert hip.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0
+    finally:
+        store.end_capture(discard=True)
+    return nodes.value

@@ -474,6 +474,11 @@ def test_bench_names_the_update_shapes_the_library_launches():
     sys.path.insert(0, REPO)
     import bench
     assert bench.CACHED_GRAD_BYTES == bound
+    m = re.search(r"constexpr uint64_t kCachedCopyElems = (\d+)ull << (\d+);", src)
+    assert m and bench.CACHED_COPY_ELEMS == int(m.group(1)) << int(m.group(2))
+    built = subprocess.run(["nm", "-C", os.path.join(REPO, "tt-perf_amd", "lib",
+                                                     "libttperf_hip.so")],
+                           capture_output=True, text=True, check=True).stdout
     big = 1 << 30
     # (optimizer, mode, layout, shape constant, master stride of an SGD form)
     for (opt, mode, layout, name, stride) in (
@@ -489,19 +494,26 @@ def test_bench_names_the_update_shapes_the_library_launches():
         e, lanes, it = shape(name)
         kname = "adam" if opt == "adamw" else "sgd"
         tmpl = f"{grad_t}, {mixed_t}, " + (f"{stride}, " if stride else "")
-        want = f"{kname}_lane_kernel<{tmpl}{e}, {lanes}, {it}>"
+        copy_nt = ", true" if opt == "adamw" else ""
+        want = f"{kname}_lane_kernel<{tmpl}{e}, {lanes}, {it}{copy_nt}>"
         assert bench.update_kernel_name(opt, mode, big, layout) == want, (opt, mode, layout)
+        assert f" ttp::{want}(" in built, want
         # below the bound: MIXED Adam its cached-gradient lane shape, MIXED SGD momentum in
         # the default layout the four-element kernel, every other update the same lane form
         if name == "AdamMixed":
             e, lanes, it = shape("AdamMixedCached")
-            want = f"adam_lane_kernel<{tmpl}{e}, {lanes}, {it}>"
+            want = f"adam_lane_kernel<{tmpl}{e}, {lanes}, {it}, true>"
+            line = bench.CACHED_COPY_ELEMS
+            assert bench.update_kernel_name(opt, mode, line + 1, layout) == want
+            assert f" ttp::{want}(" in built, want
+            want = f"adam_lane_kernel<{tmpl}{e}, {lanes}, {it}, false>"
+            assert bench.update_kernel_name(opt, mode, line, layout) == want
         if name == "SgdMixed":
             want = f"sgd_kernel<{grad_t}, {mixed_t}, {stride}>"
         assert bench.update_kernel_name(opt, mode, 1 << 20, layout) == want, (opt, mode, layout)
-        # and the library launches that instantiation
-        kern = re.sub(r"<.*", "", want)
-        assert kern in src
+        # and the library holds that instantiation
+        assert f" ttp::{want}(" in built, want
+    assert f" ttp::{bench.update_kernel_name('sgd', 'bf16', big)}(" in built
     # the library launches no four-element Adam kernel, and the four-element SGD kernel only
     # in mixed precision
     assert "adam_kernel<" not in src

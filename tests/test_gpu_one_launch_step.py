@@ -3,10 +3,9 @@ update), which per-kernel timing selects: the same stores, gradients and options
 bits in every buffer, the step state and the report.  Tables end inside a lane's vector, a wave's
 part, a tile and a chunk, and sit at and beyond the one-launch step's limits (64 tiles, 32,768
 elements)."""
-import numpy as np
 import pytest
 
-from gpu_util import torch_mod
+from gpu_util import captured_launches, torch_mod
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +93,34 @@ def test_same_bits_as_the_general_step(mode, layout, opt, table):
         store.close()
     assert repr(pair[0][0]) == repr(pair[1][0])
     assert pair[0][1] == pair[1][1]
+
+
+@pytest.mark.parametrize("opt", list(OPTS))
+@pytest.mark.parametrize("mode,layout", [("fp32", "default"), ("mixed", "default"),
+                                         ("mixed", "sgd"), ("bf16", "default")])
+def test_which_steps_are_one_launch(mode, layout, opt):
+    """At the limits one launch, just beyond them a norm pass and an update; so with per-kernel
+    timing and with the norm from per-tensor sums."""
+    import ttperf
+    if (mode == "bf16" and opt != "sgd") or (layout == "sgd" and opt.startswith("adam")):
+        pytest.skip("not a step of this store")
+    torch = torch_mod()
+    call, hp = OPTS[opt]
+    for table, sizes in TABLES.items():
+        store = ttperf.ParamStore([(n,) for n in sizes], mode=mode, layout=layout)
+        store.torch_view(ttperf.BUF_GRAD).normal_(0, 1.0)
+        torch.cuda.synchronize()
+        store.mark_grads()
+        getattr(store, call)(**dict(hp, max_grad_norm=1.0))  # state and tables are there
+
+        def launches(**kw):
+            return captured_launches(store, lambda: getattr(store, call)(**dict(hp, **kw)))
+
+        general = 2 if table in ("beyond", "65 tensors") else 1
+        assert launches(max_grad_norm=1.0) == general, table
+        store.timing(True)
+        assert launches(max_grad_norm=1.0) == 2, table
+        store.timing(False)
+        store.grad_sumsq_tensors()
+        assert launches(max_grad_norm=1.0, tensor_sums=True) == 2, table
+        store.close()

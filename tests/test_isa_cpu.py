@@ -89,7 +89,9 @@ def test_every_kernel_is_in_the_assembly(isa):
     text = "\n".join(isa["ttperf.s"])
     for k in ("adam_lane_kernel", "sgd_lane_kernel", "norm_partials_kernel",
               "norm_finalize_kernel", "accumulate_grad_tiles_kernel",
-              "combine_pending_sums_kernel", "tensor_sums_kernel"):
+              "combine_pending_sums_kernel", "tensor_sums_kernel", "adam_small_kernel",
+              "sgd_small_kernel", "sgd_bf16_small_kernel", "swap_step_kernel",
+              "gather_slot4_kernel", "scatter_slot4_kernel"):
         assert re.search(r"^_ZN3ttp\d+" + k, text, re.M), k
 
 
