@@ -36,6 +36,8 @@ def _torch_storages(tensors):
     import torch
     if torch.cuda.get_allocator_backend() == "pluggable":
         return None
+    if len(tensors) == 1:  # (as below, 0.6 us sooner)
+        return tensors if tensors[0].untyped_storage().resizable() else None
     storages = dict(zip(map(torch.Tensor.untyped_storage, tensors), tensors))
     if not all(map(torch.UntypedStorage.resizable, storages)):
         return None
