@@ -6,8 +6,8 @@
  * exp_avg_sq, momentum); the optimizer-private fp32 state is interleaved in records of
  * 64-element slots (see ttp_buffer_layout).  A step over all tensors is one multi-tensor update
  * launch (split in several only beyond 2^32 work-items), plus, when clipping or loss scaling
- * is on, a grad-norm/inf-check pass (one launch, two above 256 MiB of gradients); over a small
- * set both are one launch.
+ * is on, a grad-norm/inf-check pass (one launch, two above 256 MiB of gradients) that also takes
+ * the step's decisions; over a small set both are one launch.
  *
  * Reference interfaces each group of entry points replaces (csirak/tt-perf):
  *   ttp_create / ttp_destroy / ttp_tensor_*  — per-parameter storage owned by
@@ -479,12 +479,12 @@ int ttp_graph_launch(ttp_graph* graph);
 int ttp_graph_destroy(ttp_graph* graph);
 
 /* ---- per-kernel timing (HIP events on the context's stream) ------------------------------ */
-#define TTP_KERNEL_NORM 0   /* grad-norm / inf-check / scaler finalize pass */
+#define TTP_KERNEL_NORM 0   /* grad-norm / inf-check pass and the step's decisions */
 #define TTP_KERNEL_UPDATE 1 /* fused multi-tensor update pass               */
 /* on = 1 starts recording an event pair around every launch of every kernel. */
 int ttp_timing_enable(ttp_ctx* ctx, int on);
 /* Waits for the recorded events, returns the summed milliseconds and the count of `kernel`
- * passes since the last reset (an event pair spans each pass: a norm pass with its finalize,
+ * passes since the last reset (an event pair spans each pass: a norm pass with its decisions,
  * an update with all its launches), then forgets them. */
 int ttp_timing_collect(ttp_ctx* ctx, int kernel, double* total_ms, uint64_t* launches);
 

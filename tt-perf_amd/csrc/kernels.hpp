@@ -1,7 +1,9 @@
 // kernels.hpp — gfx950 device code of libttperf_hip.
 //
 // One optimizer step over a small tensor set is one launch (see adam_small_kernel); over any
-// other, at most three on one stream:
+// other, at most three on one stream (an update of more than 2^32 work-items is split, and
+// mark_mom_init_kernel follows a momentum step whose decisions did not set the marks: of more
+// than 4096 tensors, or without decisions on the device):
 //   norm_partials_kernel  reads only the gradients (2 B/param bf16, 4 B/param fp32) in 16 KiB
 //                         tiles: fp64 sum of squares of the unscaled grads, one partial per
 //                         block; the last block to finish sums the partials in index order
@@ -257,8 +259,8 @@ struct FinalizeArgs {
 // its first one where the decisions mark it (the update that follows must still see that it is
 // the first), 1 from then on.  Any mark but 0 means a buffer that holds a value to every step
 // that does not stage its marks.  (Marked in a launch after the update, a loss-scaled SGD momentum
-// step took 13.1 us at 1.0M parameters and takes 10.4; nanoGPT-char 44.5 and 43.1; GPT-2 124M 413.7
-// and 412.0.)
+// step took 13.1 us at 1.0M parameters and takes 10.4; nanoGPT-char 44.5 and 43.1; at GPT-2 124M,
+// 414 us, the two do not differ beyond noise.)
 constexpr uint32_t kMomNew = 2u;
 
 // torch _amp_update_scale_ semantics, over this step's overflow and the pending overflow of
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(kBlock) void norm_partials_kernel(const GradT* __re
     for (; c < t1; c += gridDim.x) {
         const R* q = reinterpret_cast<const R*>(g + ch.begin) + threadIdx.x;
         const uint32_t count = ch.count;
-        const uint32_t next = c + gridDim.x;  // (at most 2^28 tiles, 2^17 blocks: no wrap)
+        const uint32_t next = c + gridDim.x;  // (below 2^28 tiles, 2^24 blocks: no wrap)
         ch = load_chunk(tiles, next < t1 ? next : c);
         if (count == kTile) {
             R w[kNormLoads];

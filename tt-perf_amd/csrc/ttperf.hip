@@ -15,8 +15,9 @@
 //     tensors is built once; a second table is built only while some tensor has no grad
 //     (py/optim.py:56-57 skip);
 //   * step: [norm pass, whose last block decides, when clipping or loss scaling] + one fused
-//     update pass (one launch for both over small tensor sets), all on the context's stream, no host synchronisation (the skip decision
-//     and, with loss scaling, the step count live on the device).
+//     update pass (one launch for both over small tensor sets), all on the context's stream, no
+//     host synchronisation (the skip decision and, with loss scaling, the step count live on the
+//     device).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1189,8 +1190,8 @@ void release(ttp_ctx* c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (void* p : {(void*)c->grad, (void*)c->records, (void*)c->momentum, (void*)c->mom_init,
-                    (void*)c->st, (void*)c->slots, (void*)c->partials, (void*)c->tickets, c->staging, (void*)c->tsum,
-                    (void*)c->tile_sums, (void*)c->acc_tiles, (void*)c->tile_base,
+                    (void*)c->st, (void*)c->slots, (void*)c->partials, (void*)c->tickets,
+                    c->staging, (void*)c->tsum, (void*)c->tile_sums, (void*)c->acc_tiles, (void*)c->tile_base,
                     (void*)c->tsum_pending})
         if (p) (void)hipFree(p);
     for (auto& kv : c->bias_tables) (void)hipFree(kv.second.first);
