@@ -52,7 +52,13 @@ def bench(monkeypatch):
     names = ("ttp_download", "ttp_upload", "ttp_accumulate_grad", "ttp_accumulate_grad_multi", "ttp_sync",
              "ttp_destroy")
     lib = types.SimpleNamespace(**{n: entry(n) for n in names})
-    lib.ttp_get_stream = lambda h, out: asked.append("ttp_get_stream") or 0
+
+    def get_stream(h, out):
+        asked.append("ttp_get_stream")
+        out._obj.value = st.moved_to
+        return 0
+
+    lib.ttp_get_stream = get_stream
     asked = []
     monkeypatch.setattr(S.L, "lib", lib)
     stream = types.SimpleNamespace(synchronize=lambda: log.append("torch waits"),
@@ -64,7 +70,7 @@ def bench(monkeypatch):
     st._h, st.mode, st.device, st._in_capture = None, S.L.MODE_FP32, 0, False
     st.tensors = [S.Tensor(st, i, (N,)) for i in range(3)]
     st.total = 3 * N
-    st.asked = asked
+    st.asked, st.moved_to = asked, 0
     st._stream_handle = 0  # adopted: the store's stream and torch's are both the default one
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     return st, log
@@ -117,3 +123,19 @@ def test_a_store_on_its_own_stream_asks_nothing(bench, entry):
     else:
         _call(st, entry, [src])
     assert log[0] == "torch waits" and log[2:] == ["ttp_sync"] and not st.asked
+
+
+def test_a_stream_set_behind_the_stores_back_is_not_taken_for_torchs(bench):
+    """ttp_set_stream called on the store's handle: the library's answer counts."""
+    st, log = bench
+    st.moved_to = 8
+    _call(st, "accumulate", [_tensor("torch").as_subclass(_Device)])
+    assert log == ["torch waits", "ttp_accumulate_grad", "ttp_sync"] and st.asked
+
+
+def test_nothing_is_left_unread_while_torch_captures(bench, monkeypatch):
+    """The store's call waits, which a capture refuses."""
+    st, log = bench
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    _call(st, "upload", [_tensor("torch").as_subclass(_Device)])
+    assert log == ["torch waits", "ttp_upload", "ttp_sync"]
