@@ -12,7 +12,6 @@ from __future__ import annotations
 
 import ctypes as C
 import gc
-import itertools
 import math
 import operator
 import weakref
@@ -485,10 +484,9 @@ class ParamStore(_StepSlots):
         if kept is None:
             self.sync()
             return
-        import torch
         stream, keep = kept
-        for _ in map(torch.Tensor.record_stream, keep, itertools.repeat(stream)):
-            pass
+        for t in keep:
+            t.record_stream(stream)
 
     def _check_captured_tensor(self, t, n, which):
         """While capturing, a device transfer becomes a copy node that reads or writes `t`'s
